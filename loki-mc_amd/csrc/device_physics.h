@@ -351,6 +351,14 @@ __device__ __forceinline__ V cos_chi(const DevProcesses& pr, int p, V energy, V 
     }
 }
 
+// sin(chi) of a sampled cos(chi).  A sampler can round past 1: the FP32
+// screened-Coulomb quotient (sp + 1 - (2 sp + 1) R) / (sp + 1 - R) at R = 0 is
+// x / x, which an FP32 division of a few ulp need not make 1; that is a
+// scattering angle of 0, not a negative square.
+template <typename V> __device__ __forceinline__ V sin_chi(V cosChi) {
+    return sqrt(fmax((V)1 - cosChi * cosChi, (V)0));
+}
+
 template <typename V> struct Sph { V norm, sinT, cosT, sinP, cosP; };
 
 // MathFunctions::cart2sph (MathFunctions.C:143-163)
@@ -569,7 +577,7 @@ __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron
         double relAfter = relE - loss;
         if (relAfter <= 0) { o.pid = -1; return; }
         V cc = cos_chi<V>(pr, chosen, (V)relE, (V)relAfter, rng, 6);
-        V sc = sqrt((V)1 - cc * cc);
+        V sc = sin_chi(cc);
         V se, ce;
         turn_sincos(rng.u(7), se, ce);
         V u[3];
@@ -611,7 +619,7 @@ __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron
     V cc;
     if (boeuf) cc = sqrt(scE / net);
     else cc = cos_chi<V>(pr, chosen, inc, scE, rng, 6);
-    const V sc = sqrt((V)1 - cc * cc);
+    const V sc = sin_chi(cc);
     V se, ce;
     turn_sincos(rng.u(7), se, ce);
     V u[3];
@@ -634,11 +642,11 @@ __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron
     // the ejected electron (ionizationCollision, BoltzmannMC.C:1228-1267)
     V cCe, sCe, sEe, cEe;
     if (boeuf) {
-        cCe = sqrt(ej / net); sCe = sqrt((V)1 - cCe * cCe);
+        cCe = sqrt(ej / net); sCe = sin_chi(cCe);
         sEe = -se; cEe = -ce;
     } else {
         cCe = cos_chi<V>(pr, chosen, inc, ej, rng, 9);
-        sCe = sqrt((V)1 - cCe * cCe);
+        sCe = sin_chi(cCe);
         turn_sincos(rng.u(10), sEe, cEe);
     }
     euler(sCe, cCe, sEe, cEe, s, u);

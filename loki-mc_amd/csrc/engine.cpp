@@ -246,8 +246,9 @@ public:
     // device buffers
     DevBuf<RecA<V>> recA;  // electron records (FP64: their sampled part)
     DevBuf<RecB<V>> recB;  // FP64: the draw part of the records
-    DevBuf<uint32_t> holeList, markKeys, status, queue;
-    DevBuf<uint8_t> alive;
+    DevBuf<uint32_t> holeList, status, queue;
+    DevBuf<CondPop> pop;
+    DevBuf<uint8_t> alive, laneMarks;
     DevBuf<V> tables;
     DevBuf<CondParams> dconds;
     DevBuf<Chunk> chunks;
@@ -305,7 +306,7 @@ public:
             if (timer.start[k]) (void)hipEventDestroy(timer.start[k]);
             if (timer.stop[k]) (void)hipEventDestroy(timer.stop[k]);
         }
-        recA.release(); recB.release(); holeList.release(); markKeys.release(); status.release(); queue.release();
+        recA.release(); recB.release(); holeList.release(); pop.release(); laneMarks.release(); status.release(); queue.release();
         alive.release(); tables.release(); dconds.release(); chunks.release(); holesC.release();
         surplusC.release(); markC.release(); flist.release(); phaseRow.release(); cylFlag.release();
         holeOff.release(); surOff.release(); markOff.release(); mainBase.release(); tailC.release();
@@ -503,7 +504,6 @@ public:
         if (split_record<V>()) HIP_TRY(recB.alloc(capacity));
         HIP_TRY(alive.alloc(capacity));
         HIP_TRY(holeList.alloc(capacity));
-        HIP_TRY(markKeys.alloc(capacity));
         HIP_TRY(hipMemsetAsync(alive.p, 0, capacity, stream));
         HIP_TRY(tables.alloc((size_t)n * table_block_size(I, P)));
         HIP_TRY(dconds.alloc(n));
@@ -515,14 +515,17 @@ public:
         HIP_TRY(hipMemsetAsync(holesC.p, 0, nChunks * sizeof(int32_t), stream));
         HIP_TRY(hipMemsetAsync(surplusC.p, 0, nChunks * sizeof(int32_t), stream));
         HIP_TRY(hipMemsetAsync(markC.p, 0, nChunks * sizeof(int32_t), stream));
+        HIP_TRY(laneMarks.alloc((size_t)nChunks * kWave));
+        dw.popStride = (n + 7) / 8 * 8;  // 16-byte totals, 128-byte lines
+        HIP_TRY(pop.alloc((size_t)kPopCopies * dw.popStride));
+        HIP_TRY(hipMemsetAsync(pop.p, 0, pop.n * sizeof(CondPop), stream));
         recSize = event_record_size(P);
         summarySize = recSize + kMomentRecord + 8;
         HIP_TRY(tailC.alloc((size_t)nChunks * CT_SIZE));
         HIP_TRY(momC.alloc((size_t)nChunks * kMomentRecord));
         HIP_TRY(hipMemsetAsync(tailC.p, 0, (size_t)nChunks * CT_SIZE * sizeof(double), stream));
-        // reduction groups of at most kFinishGroup work units, when a condition
-        // has more units than one block reduces quickly (one condition of 1e8
-        // electrons: 98,000 units, 1.3 ms in one block)
+        // reduction groups, when a condition has more units than one block
+        // reduces quickly (one condition of 1e8 electrons: 98,000 units)
         {
             int maxCh = 0;
             for (int c = 0; c < n; ++c) maxCh = std::max(maxCh, (int)hcp[c].nChunks);
@@ -530,10 +533,11 @@ public:
                 std::vector<int32_t> gc, gf, gn, cg(n), cn(n);
                 for (int c = 0; c < n; ++c) {
                     cg[c] = (int32_t)gc.size();
-                    for (int j = 0; j < hcp[c].nChunks; j += kFinishGroup) {
+                    const int each = std::max(kFinishGroup, (int)std::ceil(std::sqrt((double)hcp[c].nChunks)));
+                    for (int j = 0; j < hcp[c].nChunks; j += each) {
                         gc.push_back(c);
                         gf.push_back(hcp[c].chunkBegin + j);
-                        gn.push_back(std::min(kFinishGroup, (int)hcp[c].nChunks - j));
+                        gn.push_back(std::min(each, (int)hcp[c].nChunks - j));
                     }
                     cn[c] = (int32_t)gc.size() - cg[c];
                 }
@@ -653,13 +657,18 @@ public:
         ds = DevState<V>{recA.p, recB.p, alive.p};
         dw.conds = dconds.p; dw.chunks = chunks.p; dw.holesC = holesC.p; dw.surplusC = surplusC.p;
         dw.markC = markC.p; dw.holeOff = holeOff.p; dw.surOff = surOff.p; dw.markOff = markOff.p;
-        dw.holeList = holeList.p; dw.markKeys = markKeys.p; dw.tailC = tailC.p; dw.momC = momC.p; dw.accCount = accCount.p;
+        dw.holeList = holeList.p; dw.laneMarks = laneMarks.p; dw.pop = pop.p; dw.tailC = tailC.p; dw.momC = momC.p; dw.accCount = accCount.p;
         dw.accGain = accGain.p; dw.accLoss = accLoss.p; dw.plans = plans.p;
         dw.status = status.p; dw.queue = queue.p; dw.summary = summary.p; dw.summarySize = summarySize;
         dw.recSize = recSize; dw.nChunks = nChunks; dw.nCond = n;
         dw.groupCond = gCond.p; dw.groupFirst = gFirst.p; dw.groupCount = gCount.p;
         dw.condGroup = cGroup.p; dw.condGroups = cGroups.p; dw.tailG = tailG.p; dw.momG = momG.p;
         dw.nGroups = nGroups;
+        dw.planMarks = dw.planPairs = 0;
+        for (int c = 0; c < n; ++c) {
+            if (hcp[c].nMain > kPlanDirect) dw.planMarks = 1;
+            if (hcp[c].nChunks > kPairsDirect) dw.planPairs = 1;
+        }
         dh.eedf = hEedf.p; dh.eedfPer = hPer.p; dh.eadf = hEadf.p; dh.evdf = hEvdf.p; dh.grid = grid.p;
         dh.evdf3 = hEvdf3.p; dh.n3 = n3;
         dh.phaseRow = phaseRow.p; dh.cyl = cylFlag.p;
@@ -865,14 +874,14 @@ public:
     ekmc_status launch_cycle() {
         if (!useGraph || timer.level >= 2) {
             HIP_TRY(launch_popctl<V>(ds, dw, stream));
-            HIP_TRY(launch_sample<V>(ds, dw, stream));
+            HIP_TRY(launch_settle<V>(ds, dw, stream));
             HIP_TRY(launch_reduce());
             return EKMC_OK;
         }
         if (!cycExec) {
             HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
             hipError_t e = launch_popctl<V>(ds, dw, stream);
-            if (e == hipSuccess) e = launch_sample<V>(ds, dw, stream);
+            if (e == hipSuccess) e = launch_settle<V>(ds, dw, stream);
             if (e == hipSuccess) e = launch_reduce();
             hipGraph_t g = nullptr;
             const hipError_t ec = hipStreamEndCapture(stream, &g);
@@ -1124,7 +1133,7 @@ public:
         HIP_TRY(hipMemcpyAsync(dconds.p, hcp.data(), nCond * sizeof(CondParams), hipMemcpyHostToDevice, stream));
         set_kernel_timer(&timer);
         HIP_TRY(launch_init<V>(ds, dw, totalMain, mainBase.p, thermalDev.p, stream));
-        HIP_TRY(launch_sample<V>(ds, dw, stream));
+        HIP_TRY(launch_settle<V>(ds, dw, stream));
         HIP_TRY(launch_reduce());
         ekmc_status st = wait_summary();
         if (st != EKMC_OK) return st;

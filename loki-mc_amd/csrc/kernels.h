@@ -66,8 +66,8 @@ template <typename V> __host__ __device__ inline auto& draw_part(Rec<V>& q) {
 template <typename V> struct DevState {
     RecA<V>* ra;      // [pool capacity]
     RecB<V>* rb;      // [pool capacity] FP64 form only
-    uint8_t* alive;   // [pool capacity] 0 dead/empty, 1 alive, 2 clone made by this interval's
-                      // population control (back to 1 in the sampling kernel)
+    uint8_t* alive;   // [pool capacity] 0 dead/empty, 1 alive, 2 or 3 (by the parity of the interval)
+                      // filled by population control (back to 1 in the next interval's k_settle)
 };
 
 // A wave's unit of work: up to `count` main electrons of one condition plus
@@ -85,18 +85,31 @@ struct Chunk {
 // Per-chunk scalar tallies (FP64, reduced in chunk order).
 enum ChunkTail { CT_FIELD = 0, CT_NULL, CT_REAL, CT_EVENTS, CT_ESCAPE, CT_MAXE, CT_GROWTH, CT_PAD, CT_SIZE };
 
+// Totals of one condition's population control in an interval: added up by the
+// waves of its chunks, cleared by k_finish.
+struct CondPop {
+    uint32_t holes, surplus;  // after the flights (holes not refilled by the chunk, newborns left)
+    uint32_t marks;           // removal marks
+    uint32_t holesAfter;      // after removals: holes, and as many newborns
+};
+
+constexpr int kPopCopies = 8;
+
 // Device work buffers shared by the interval kernels.
 struct DevWork {
     const CondParams* conds;      // [n_cond]
     const Chunk* chunks;          // [n_chunks]
     int32_t* holesC;              // [n_chunks] holes left after the chunk's own refill
     int32_t* surplusC;            // [n_chunks] newborns left in the chunk's region
-    int32_t* markC;               // [n_chunks]
-    int64_t* holeOff;             // [n_chunks] exclusive offsets within the condition
+    int32_t* markC;               // [n_chunks] marks of the chunk
+    uint8_t* laneMarks;           // [64 n_chunks] marks of each lane of the chunk (255: more than 254)
+    CondPop* pop;                 // [kPopCopies * popStride] totals of the interval's population control
+    int popStride;                // n_cond rounded up to whole cache lines
+    int64_t* holeOff;             // [n_chunks] exclusive offsets within the condition (k_plan_pairs)
     int64_t* surOff;
-    int64_t* markOff;
+    int64_t* markOff;             // (k_plan_marks)
+    int planMarks, planPairs;     // a condition needs k_plan_marks / k_plan_pairs
     uint32_t* holeList;           // [pool capacity]; a chunk's holes at holeList[first ..)
-    uint32_t* markKeys;           // [pool capacity]; removal keys of a condition's marks at [base ..)
     double* tailC;                // [n_chunks * CT_SIZE]
     double* momC;                 // [n_chunks * kMomentRecord]
     unsigned long long* accCount; // [n_cond * P] real collisions per process
@@ -123,8 +136,18 @@ struct DevWork {
     double* momG;                 // [nGroups * kMomentRecord]
     int nGroups;
 };
-constexpr int kFinishDirect = 4096;  // work units a condition reduces directly
-constexpr int kFinishGroup = 2048;   // work units per reduction group
+// A block of k_finish sums 28 records at a time; for a condition of more than
+// 448 work units (16 turns) a group kernel, with about as many groups as units
+// per group, shortens both sums (925 units: 21 us in one block, 14 us in
+// two steps; 261 units: 9.3 us against 11.8).
+constexpr int kFinishDirect = 448;
+constexpr int kFinishGroup = 64;     // fewest work units per reduction group
+// Conditions of at most this many electrons have their removal threshold
+// worked out by every block of k_apply_marks (plans_direct).
+constexpr int64_t kPlanDirect = 32768;
+// Conditions of at most this many chunks have the pairs of holes and newborns
+// found in the per-chunk counts (wave_locate): 8 tiles of 512 counts at most.
+constexpr int kPairsDirect = 4096;
 
 // A contiguous range of main slots of one condition (histogram blocks).
 struct SlotRange {
@@ -199,11 +222,12 @@ hipError_t launch_init(const DevState<V>& s, const DevWork& w, int64_t totalMain
 template <typename V>
 hipError_t launch_flights(const DevState<V>& s, const DevWork& w, const DevProcesses& pr,
                           const V* tables, const DevHist& h, const FlightLists& fl, hipStream_t st);
-// Population control after the flights: the same launches every interval.
+// Removals after the flights: the same launches every interval.
 template <typename V>
 hipError_t launch_popctl(const DevState<V>& s, const DevWork& w, hipStream_t st);
+// Pairs, clones and the ensemble sums.
 template <typename V>
-hipError_t launch_sample(const DevState<V>& s, const DevWork& w, hipStream_t st);
+hipError_t launch_settle(const DevState<V>& s, const DevWork& w, hipStream_t st);
 template <typename V>
 hipError_t launch_hist(const DevState<V>& s, const DevHist& h, hipStream_t st);
 hipError_t launch_finish(const DevWork& w, int P, hipStream_t st);
@@ -232,8 +256,7 @@ hipError_t launch_op_philox(int64_t n, const uint32_t* ctr, const uint32_t* key,
                             hipStream_t st);
 
 // kernel names for timing (index matches the event slots used by the engine)
-enum KernelId { K_INIT = 0, K_ADVANCE, K_PLAN, K_MARKS, K_APPLY, K_PAIRS, K_MOVE, K_CLONE, K_SAMPLE,
-                K_HIST, K_REDUCE, K_COUNT };
+enum KernelId { K_INIT = 0, K_ADVANCE, K_MARKS, K_APPLY, K_SETTLE, K_HIST, K_REDUCE, K_COUNT };
 extern const char* kKernelNames[K_COUNT];
 // Per-kernel HIP events recorded by the launchers when set.
 struct KernelTimer {

@@ -11,18 +11,16 @@
 //                  Collisions are counted in LDS per wave and added to the
 //                  condition's integer accumulators; attached electrons leave
 //                  holes that the chunk's own newborns refill.
-//   k_plan         per condition: scans of holes/surplus over its chunks, the
-//                  population M, removals R or clones C.
-//   k_marks / k_plan_marks / k_apply_marks
-//                  exact uniform removal of R electrons: Bernoulli marks drawn
-//                  by geometric skips, then the R marks with the smallest
-//                  random keys (radix select) are removed.
-//   k_plan_pairs / k_move / k_clone
-//                  surplus newborns fill holes; clones of uniformly chosen
+//   k_marks        exact uniform removal of R electrons, first half: Bernoulli
+//                  marks drawn by geometric skips, counted per chunk.
+//   k_apply_marks  second half: the R marks with the smallest random keys are
+//                  removed.  (k_plan_marks finds the R-th smallest key of a
+//                  large condition, k_plan_pairs the hole and newborn offsets
+//                  of a condition of very many chunks, one block each.)
+//   k_settle       surplus newborns fill holes; clones of uniformly chosen
 //                  electrons fill the holes that remain (rejection, as the
-//                  reference does at BoltzmannMC.C:1368-1371).
-//   k_sample       FP64 moments of the N electrons at t_sync, per chunk
-//                  (BoltzmannMC.C:1410-1482).
+//                  reference does at BoltzmannMC.C:1368-1371); FP64 moments of
+//                  the N electrons at t_sync, per chunk (BoltzmannMC.C:1410-1482).
 //   k_finish       per condition: fixed-order sums of the chunk records, the
 //                  integer accumulators, the plan; resets the queues.
 // Every floating-point reduction runs in a fixed order (wave butterflies, then
@@ -33,8 +31,7 @@
 
 namespace ekmc {
 
-const char* kKernelNames[K_COUNT] = {"init", "advance", "plan", "marks", "apply_marks",
-                                     "plan_pairs", "move", "clone", "sample", "hist", "finish"};
+const char* kKernelNames[K_COUNT] = {"init", "advance", "marks", "apply_marks", "settle", "hist", "finish"};
 
 static KernelTimer* g_timer = nullptr;
 void set_kernel_timer(KernelTimer* t) { g_timer = t; }
@@ -269,6 +266,25 @@ template <typename V> __device__ __forceinline__ void ring_read(const lds_uint4*
     rec_to_electron(q, e);
 }
 
+// -------------------------------------------- population-control totals
+// A condition's totals: the waves of its chunks add to kPopCopies copies, by
+// block index, so to different addresses on different XCDs (blocks go to the
+// XCDs in turn).  Adds to one address from all of them take 8 ns each: with
+// one copy, the 98,000 chunks of one condition of 1e8 electrons made k_marks
+// 0.81 ms instead of 0.08 ms.
+__device__ __forceinline__ CondPop& pop_mine(const DevWork& w, int c) {
+    return w.pop[(size_t)(blockIdx.x % kPopCopies) * w.popStride + c];
+}
+__device__ __forceinline__ CondPop pop_total(const DevWork& w, int c) {
+    CondPop t = {};
+#pragma unroll
+    for (int k = 0; k < kPopCopies; ++k) {
+        const CondPop p = w.pop[(size_t)k * w.popStride + c];
+        t.holes += p.holes; t.surplus += p.surplus; t.marks += p.marks; t.holesAfter += p.holesAfter;
+    }
+    return t;
+}
+
 // ------------------------------------------------------- block helpers
 // Sum over a kBlock-thread block in a fixed order; result valid in thread 0.
 __device__ double block_sum(double v, double* red) {
@@ -440,7 +456,7 @@ __device__ void wave_refill(const DevState<V>& s, uint32_t* holeList, const Chun
         used += __popcll(am);
     }
     const int filled = used < holes ? used : holes;
-    for (int b = filled; b < holes; b += kWave) {  // remaining holes to the list front
+    for (int b = filled; filled > 0 && b < holes; b += kWave) {  // remaining holes to the list front
         const int h = b + lane;
         uint32_t v = 0;
         if (h < holes) v = holeList[ch.first + h];
@@ -707,6 +723,8 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
     if (lane == 0) {
         w.holesC[cid] = holes;
         w.surplusC[cid] = remaining;
+        if (holes) atomicAdd(&pop_mine(w, c).holes, (uint32_t)holes);
+        if (remaining) atomicAdd(&pop_mine(w, c).surplus, (uint32_t)remaining);
         double* t = w.tailC + (size_t)cid * CT_SIZE;
         t[CT_FIELD] = fg;
         t[CT_NULL] = (double)nn;
@@ -783,23 +801,34 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_w
 }
 
 // ------------------------------------------------------ population control
-__global__ __launch_bounds__(1024) void k_plan(DevWork w) {
-    __shared__ int64_t lds[1024];
-    const int c = blockIdx.x;
-    const CondParams cp = w.conds[c];
-    if (!cp.active) return;
-    const int64_t H = block_exclusive_scan(w.holesC + cp.chunkBegin, w.holeOff + cp.chunkBegin, cp.nChunks, lds);
-    const int64_t S = block_exclusive_scan(w.surplusC + cp.chunkBegin, w.surOff + cp.chunkBegin, cp.nChunks, lds);
-    if (threadIdx.x == 0) {
-        PopPlan pl = {};
-        pl.holes = H;
-        pl.surplus = S;
-        pl.alive = cp.nMain - H + S;
-        pl.remove = S > H ? S - H : 0;
-        const double R = (double)pl.remove;
-        pl.markProb = pl.remove > 0 ? fmin(1.0, (R + 8.0 * sqrt(R) + 20.0) / (double)pl.alive) : 0.0;
-        w.plans[c] = pl;
-    }
+// Four kernels after the flights bring every condition back to N electrons
+// and sample it: k_marks and k_apply_marks remove surplus electrons, k_settle
+// moves and clones electrons into holes and samples, k_finish reduces.  What
+// bounds them at ordinary sizes is latency: a kernel starts with cold L2s, so
+// each load that depends on another costs about 0.7 us, and a kernel that
+// does nothing about 2.5 us.  So what a planning kernel of one block per
+// condition would compute is taken from totals the waves add up (the removals),
+// or worked out again by every wave or block that needs it (offsets, removal
+// threshold) while it has little else to do.  One kernel for everything with
+// the last block of a condition planning was slower: handing values between
+// blocks of one launch costs more than a launch (12 us against 7 us for the
+// marks of one condition of 1e4 electrons).  Measured, all kernels after the
+// flights, against ten launches with planning kernels between them: one
+// condition of 1e4 electrons 55 -> 27 us, of 1e5 60 -> 36 us, the 64-condition
+// scan 322 -> 277 us.
+
+// The population of a condition after its flights: M alive, and the removals
+// that bring it back to N.
+__device__ __forceinline__ PopPlan plan_of(const CondPop& pop, const CondParams& cp) {
+    const int64_t H = pop.holes, S = pop.surplus;
+    PopPlan pl = {};
+    pl.holes = H;
+    pl.surplus = S;
+    pl.alive = cp.nMain - H + S;
+    pl.remove = S > H ? S - H : 0;
+    const double R = (double)pl.remove;
+    pl.markProb = pl.remove > 0 ? fmin(1.0, (R + 8.0 * sqrt(R) + 20.0) / (double)pl.alive) : 0.0;
+    return pl;
 }
 
 // Bernoulli(p) marks over a chunk's candidates [0, L): main slots
@@ -842,20 +871,37 @@ __device__ __forceinline__ bool mark_alive(const uint8_t* alive, const Chunk& ch
     return pos >= ch.count || alive[ch.first + pos] != 0;
 }
 
+// A condition of at most kPlanDirect electrons has its removal threshold and
+// its chunks' mark offsets worked out by every block of k_apply_marks: its
+// few hundred marks cost a block less than the launch of k_plan_marks and the
+// loads of its results.  Per interval, in the blocks against with k_plan_marks:
+// one condition of 1e4 electrons 8.3 us against 6.1 + 6.9, one of 1e5 11.6
+// against 6.4 + 6.5, eight of 1e5 at up to 500 Td (2 % newborns) 31 against
+// 10.3 + 10.3, the 64-condition scan with half of its conditions planned in the
+// blocks 67 + 18 against 30 + 17.
+__host__ __device__ __forceinline__ bool plans_direct(const CondParams& cp) { return cp.nMain <= kPlanDirect; }
+
+// The marks of each chunk of a condition with removals, counted per lane and
+// added to the condition's total.
 __global__ __launch_bounds__(kBlock) void k_marks(const uint8_t* alive, DevWork w) {
     const int lane = lane_id();
     const int cid = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
     if (cid >= w.nChunks) return;
     const Chunk ch = w.chunks[cid];
+    const int sur = w.surplusC[cid];
     const CondParams& cp = w.conds[ch.cond];
     if (!cp.active) return;
-    const PopPlan pl = w.plans[ch.cond];
+    const PopPlan pl = plan_of(pop_total(w, ch.cond), cp);
     if (pl.remove == 0) return;
-    MarkGen g(cp, ch, lane, pl.markProb, (int64_t)ch.count + w.surplusC[cid]);
+    MarkGen g(cp, ch, lane, pl.markProb, (int64_t)ch.count + sur);
     uint32_t m = 0;
     while (g.next()) m += mark_alive(alive, ch, g.pos) ? 1u : 0u;
+    w.laneMarks[(size_t)cid * kWave + lane] = (uint8_t)(m < 255u ? m : 255u);
     m = wave_sum_u(m);
-    if (lane == 0) w.markC[cid] = (int32_t)m;
+    if (lane == 0) {
+        w.markC[cid] = (int32_t)m;
+        if (m && plans_direct(cp)) atomicAdd(&pop_mine(w, ch.cond).marks, m);
+    }
 }
 
 // Key of the mark with condition-wide index j (uniform 32-bit word).
@@ -866,44 +912,32 @@ __device__ __forceinline__ uint32_t mark_key(const CondParams& cp, int64_t j) {
     return w[0];
 }
 
-// Scan of marks, then the removal threshold: of the K marks, the R with the
-// smallest (key, index) go, which is a uniform R-subset.  The R-th smallest
-// key comes from a 4-pass, 8-bit radix select; ties on that key are ordered
-// by index.
 constexpr int kTieCap = 1024;
-__global__ __launch_bounds__(1024) void k_plan_marks(DevWork w) {
-    __shared__ int64_t lds[1024];
-    __shared__ uint32_t hist[256];
-    __shared__ uint32_t ties[kTieCap];
-    __shared__ uint32_t sh[4];  // prefix, mask, need, tie count
-    const int c = blockIdx.x;
-    const CondParams cp = w.conds[c];
-    if (!cp.active) return;
-    PopPlan pl = w.plans[c];
-    if (pl.remove == 0) return;
-    const int64_t K = block_exclusive_scan(w.markC + cp.chunkBegin, w.markOff + cp.chunkBegin, cp.nChunks, lds);
-    const int64_t R = pl.remove;
-    if (K < R || K > 0xffffffffLL) {
-        if (threadIdx.x == 0) {
-            pl.marks = K;
-            pl.status |= ST_POPCTL;
-            w.plans[c] = pl;
-            atomicOr(&w.status[c], (uint32_t)ST_POPCTL);
-        }
-        return;
-    }
+constexpr int kNearCap = 2048;
+struct PopLds {
+    uint64_t near[kNearCap];  // (key, index) of the marks near the threshold
+    uint32_t hist[256], ties[kTieCap];
+    uint32_t sh[4];           // prefix, mask, need, tie count
+    uint32_t below, nNear;
+    int last;
+};
+
+// Key of the R-th smallest of K marks by a 4-pass, 8-bit radix select; ties
+// on that key are ordered by index.  Sets the plan's threshold; false when it
+// cannot.
+__device__ bool radix_threshold(PopLds& L, const CondParams& cp, int64_t K, int64_t R, PopPlan& pl) {
+    uint32_t* sh = L.sh;
+    uint32_t* hist = L.hist;
+    uint32_t* ties = L.ties;
     if (threadIdx.x == 0) { sh[0] = 0; sh[1] = 0; sh[2] = (uint32_t)R; sh[3] = 0; }
     __syncthreads();
-    uint32_t* keys = w.markKeys + cp.base;  // K <= the condition's pool slots
     for (int pass = 0; pass < 4; ++pass) {
         const int shift = 24 - 8 * pass;
         for (int i = threadIdx.x; i < 256; i += blockDim.x) hist[i] = 0;
         __syncthreads();
         const uint32_t prefix = sh[0], mask = sh[1];
         for (int64_t j = threadIdx.x; j < K; j += blockDim.x) {
-            uint32_t k;
-            if (pass == 0) { k = mark_key(cp, j); keys[j] = k; }
-            else k = keys[j];
+            const uint32_t k = mark_key(cp, j);
             if ((k & mask) == prefix) atomicAdd(&hist[(k >> shift) & 255u], 1u);
         }
         __syncthreads();
@@ -941,22 +975,14 @@ __global__ __launch_bounds__(1024) void k_plan_marks(DevWork w) {
     }
     const uint32_t T = sh[0], need = sh[2];  // R-th smallest key; its rank among keys == T
     for (int64_t j = threadIdx.x; j < K; j += blockDim.x) {
-        if (keys[j] == T) {
+        if (mark_key(cp, j) == T) {
             const uint32_t slot = atomicAdd(&sh[3], 1u);
             if (slot < kTieCap) ties[slot] = (uint32_t)j;
         }
     }
     __syncthreads();
     const uint32_t nt = sh[3];
-    if (nt > kTieCap || need < 1 || need > nt) {
-        if (threadIdx.x == 0) {
-            pl.marks = K;
-            pl.status |= ST_POPCTL;
-            w.plans[c] = pl;
-            atomicOr(&w.status[c], (uint32_t)ST_POPCTL);
-        }
-        return;
-    }
+    if (nt > kTieCap || need < 1 || need > nt) return false;
     // bitonic sort of the tied indices (padded to a power of two)
     int n2 = 1;
     while (n2 < (int)nt) n2 <<= 1;
@@ -976,52 +1002,107 @@ __global__ __launch_bounds__(1024) void k_plan_marks(DevWork w) {
             __syncthreads();
         }
     }
-    if (threadIdx.x == 0) {
-        pl.marks = K;
-        pl.thrKey = T;
-        pl.thrIndex = ties[need - 1];
-        w.plans[c] = pl;
+    pl.thrKey = T;
+    pl.thrIndex = ties[need - 1];
+    return true;
+}
+
+// The removal threshold of a condition by one block: of the K marks, the R
+// with the smallest (key, index) go, which is a uniform R-subset.  The keys
+// are uniform 32-bit words, so the R-th smallest lies within a few standard
+// deviations of 2^32 R / K: the marks below that window are counted and the few
+// hundred inside it (the standard deviation of the count is sqrt(R (K - R) /
+// K), K - R = 8 sqrt(R) + 20) ranked, in one pass over the keys.  A threshold
+// outside the window (six standard deviations) takes the radix select, which
+// needs five passes.  Every thread gets the plan's threshold, or the status.
+__device__ void removal_threshold(const CondParams& cp, int64_t K, PopPlan& pl, PopLds& L) {
+    const int64_t R = pl.remove;
+    pl.marks = K;
+    if (K < R || K > 0xffffffffLL) {
+        pl.status |= ST_POPCTL;
+        return;
     }
+    __syncthreads();
+    if (threadIdx.x == 0) { L.below = 0; L.nNear = 0; }
+    __syncthreads();
+    const double mid = 4294967296.0 * ((double)R / (double)K);
+    const double half = 4294967296.0 / (double)K * (6.0 * sqrt((double)R * (double)(K - R) / (double)K) + 8.0);
+    const uint32_t lo = (uint32_t)fmax(0.0, mid - half), hi = (uint32_t)fmin(4294967295.0, mid + half);
+    uint32_t under = 0;
+    for (int64_t j = threadIdx.x; j < K; j += blockDim.x) {
+        const uint32_t k = mark_key(cp, j);
+        if (k < lo) ++under;
+        else if (k <= hi) {
+            const uint32_t n = atomicAdd(&L.nNear, 1u);
+            if (n < kNearCap) L.near[n] = ((uint64_t)k << 32) | (uint32_t)j;
+        }
+    }
+    under = wave_sum_u(under);
+    if (lane_id() == 0) atomicAdd(&L.below, under);
+    __syncthreads();
+    const int64_t need = R - (int64_t)L.below;  // rank of the threshold among the near marks
+    const uint32_t nNear = L.nNear;
+    if (need < 1 || need > (int64_t)nNear || nNear > kNearCap) {
+        if (!radix_threshold(L, cp, K, R, pl)) pl.status |= ST_POPCTL;
+        return;
+    }
+    for (uint32_t i = threadIdx.x; i < nNear; i += blockDim.x) {
+        const uint64_t me = L.near[i];
+        uint32_t rank = 1;
+        for (uint32_t q = 0; q < nNear; ++q) rank += L.near[q] < me ? 1u : 0u;
+        if (rank == (uint32_t)need) L.last = (int)i;
+    }
+    __syncthreads();
+    const uint64_t thr = L.near[L.last];
+    pl.thrKey = (uint32_t)(thr >> 32);
+    pl.thrIndex = (int64_t)(uint32_t)thr;
+}
+
+// Mark offsets and removal threshold of the larger conditions, one block each.
+__global__ __launch_bounds__(1024) void k_plan_marks(DevWork w) {
+    __shared__ int64_t lds[2 * kWave + 1];
+    __shared__ PopLds L;
+    const int c = blockIdx.x;
+    const CondParams cp = w.conds[c];
+    if (!cp.active || plans_direct(cp)) return;
+    PopPlan pl = plan_of(pop_total(w, c), cp);
+    if (pl.remove == 0) return;
+    const int64_t K = block_exclusive_scan(w.markC + cp.chunkBegin, w.markOff + cp.chunkBegin, cp.nChunks, lds);
+    removal_threshold(cp, K, pl, L);
+    if (threadIdx.x == 0) w.plans[c] = pl;
 }
 
 // Marks in chunk order, then lane order, then position order; a mark at or
-// below the threshold is removed.  Removed main electrons become
-// holes of the chunk, then the chunk refills them from its newborns.
+// below the threshold is removed.  Removed main electrons become holes of the
+// chunk, then the chunk refills them from its newborns.
 template <typename V>
-__global__ __launch_bounds__(kBlock) void k_apply_marks(DevState<V> s, DevWork w) {
+__device__ __forceinline__ void apply_marks(const DevState<V>& s, const DevWork& w, const Chunk& ch,
+                                            const CondParams& cp, int cid, const PopPlan& pl, int sur, int holes,
+                                            int mine, int64_t offset) {
     const int lane = lane_id();
-    const int cid = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (cid >= w.nChunks) return;
-    const Chunk ch = w.chunks[cid];
-    const CondParams& cp = w.conds[ch.cond];
-    if (!cp.active) return;
-    const PopPlan pl = w.plans[ch.cond];
-    if (pl.remove == 0 || (pl.status & ST_POPCTL)) return;
-    const int sur = w.surplusC[cid];
     const int64_t L = (int64_t)ch.count + sur;
-    int mine = 0;
-    {
+    if (__ballot(mine == 255)) {  // a count that did not fit its byte: count again
+        mine = 0;
         MarkGen g(cp, ch, lane, pl.markProb, L);
         while (g.next()) mine += mark_alive(s.alive, ch, g.pos) ? 1 : 0;
     }
-    int64_t gi = w.markOff[cid] + wave_exclusive_scan(mine);
-    int holes = w.holesC[cid];
+    int64_t gi = offset + wave_exclusive_scan(mine);
     double growth = 0;
     MarkGen g(cp, ch, lane, pl.markProb, L);
-    bool more = g.next();
+    int left = mine;  // marks of this lane not yet visited
+    bool more = left > 0 && g.next();
     while (__ballot(more)) {
         bool kill = false, killMain = false;
         int64_t slot = 0;
-        if (more) {
-            if (mark_alive(s.alive, ch, g.pos)) {
-                const uint32_t k = w.markKeys[cp.base + gi];
-                if (k < pl.thrKey || (k == pl.thrKey && gi <= pl.thrIndex)) {
-                    kill = true;
-                    killMain = g.pos < ch.count;
-                    slot = killMain ? ch.first + g.pos : ch.region + (g.pos - ch.count);
-                }
-                ++gi;
+        if (more && mark_alive(s.alive, ch, g.pos)) {
+            const uint32_t k = mark_key(cp, gi);
+            if (k < pl.thrKey || (k == pl.thrKey && gi <= pl.thrIndex)) {
+                kill = true;
+                killMain = g.pos < ch.count;
+                slot = killMain ? ch.first + g.pos : ch.region + (g.pos - ch.count);
             }
+            ++gi;
+            --left;
         }
         const uint64_t km = __ballot(killMain);
         if (kill) {
@@ -1030,7 +1111,7 @@ __global__ __launch_bounds__(kBlock) void k_apply_marks(DevState<V> s, DevWork w
             if (killMain) w.holeList[ch.first + holes + lane_rank(km)] = (uint32_t)slot;
         }
         holes += __popcll(km);
-        if (more) more = g.next();
+        if (more) more = left > 0 && g.next();
     }
     int remaining = 0;
     wave_refill<V>(s, w.holeList, ch, holes, sur, remaining);
@@ -1038,114 +1119,206 @@ __global__ __launch_bounds__(kBlock) void k_apply_marks(DevState<V> s, DevWork w
     if (lane == 0) {
         w.holesC[cid] = holes;
         w.surplusC[cid] = remaining;
-        w.tailC[(size_t)cid * CT_SIZE + CT_GROWTH] += gsum;
+        if (holes) atomicAdd(&pop_mine(w, ch.cond).holesAfter, (uint32_t)holes);
+        if (gsum != 0) w.tailC[(size_t)cid * CT_SIZE + CT_GROWTH] += gsum;
     }
 }
 
+template <typename V>
+__global__ __launch_bounds__(kBlock) void k_apply_marks(DevState<V> s, DevWork w) {
+    __shared__ PopLds L;
+    __shared__ int conds[kWavesPerBlock];
+    const int lane = lane_id(), wid = threadIdx.x / kWave;
+    const int cid = blockIdx.x * kWavesPerBlock + wid;
+    const bool in = cid < w.nChunks;
+    Chunk ch = {};
+    int c = -1, sur = 0, holes = 0, mine = 0;
+    PopPlan pl = {};
+    if (in) {
+        ch = w.chunks[cid];
+        sur = w.surplusC[cid];
+        holes = w.holesC[cid];
+        mine = w.laneMarks[(size_t)cid * kWave + lane];
+        if (w.conds[ch.cond].active) {
+            pl = plan_of(pop_total(w, ch.cond), w.conds[ch.cond]);
+            if (pl.remove > 0) c = ch.cond;
+        }
+    }
+    const bool direct = c >= 0 && plans_direct(w.conds[c]);
+    if (lane == 0) conds[wid] = direct ? c : -1;
+    __syncthreads();
+    // thresholds of the block's conditions (one, but where a block ends one
+    // condition and begins the next)
+    for (int k = 0; k < kWavesPerBlock; ++k) {
+        const int cc = conds[k];
+        if (cc < 0 || (k > 0 && conds[k - 1] == cc)) continue;
+        const CondPop pop = pop_total(w, cc);
+        PopPlan q = plan_of(pop, w.conds[cc]);
+        removal_threshold(w.conds[cc], pop.marks, q, L);
+        if (c == cc) pl = q;
+        __syncthreads();
+    }
+    if (c < 0) return;
+    const CondParams& cp = w.conds[c];
+    int64_t offset;
+    if (direct) {
+        uint32_t before = 0;
+        for (int k = lane; k < ch.local; k += kWave) before += (uint32_t)w.markC[cp.chunkBegin + k];
+        offset = wave_sum_u(before);
+    } else {
+        pl = w.plans[c];
+        offset = w.markOff[cid];
+    }
+    if (pl.status & ST_POPCTL) {
+        if (lane == 0) atomicOr(&w.status[c], (uint32_t)ST_POPCTL);
+        return;
+    }
+    apply_marks<V>(s, w, ch, cp, cid, pl, sur, holes, mine, offset);
+}
+
+// Offsets of the holes and surplus newborns of the conditions with more than
+// kPairsDirect chunks, one block each.  (k_settle finds the pairs of the
+// others in the per-chunk counts.)
 __global__ __launch_bounds__(1024) void k_plan_pairs(DevWork w) {
-    __shared__ int64_t lds[1024];
+    __shared__ int64_t lds[2 * kWave + 1];
     const int c = blockIdx.x;
     const CondParams cp = w.conds[c];
-    if (!cp.active) return;
-    PopPlan pl = w.plans[c];
-    if (pl.holes == 0 && pl.surplus == 0) return;
-    const int64_t H = block_exclusive_scan(w.holesC + cp.chunkBegin, w.holeOff + cp.chunkBegin, cp.nChunks, lds);
-    const int64_t S = block_exclusive_scan(w.surplusC + cp.chunkBegin, w.surOff + cp.chunkBegin, cp.nChunks, lds);
-    if (threadIdx.x == 0) {
-        pl.holes = H;
-        pl.surplus = S;
-        w.plans[c] = pl;
-    }
+    if (!cp.active || cp.nChunks <= kPairsDirect) return;
+    const CondPop pop = pop_total(w, c);
+    if (pop.holes == 0 && pop.surplus == 0) return;
+    block_exclusive_scan(w.holesC + cp.chunkBegin, w.holeOff + cp.chunkBegin, cp.nChunks, lds);
+    block_exclusive_scan(w.surplusC + cp.chunkBegin, w.surOff + cp.chunkBegin, cp.nChunks, lds);
 }
 
-// Pair i (i < min(H, S)): hole i of the condition <- surplus newborn i.  The
-// waves of a condition's chunks stride over the pairs.
-template <typename V>
-__global__ __launch_bounds__(kBlock) void k_move(DevState<V> s, DevWork w) {
+// Chunk and place within it of every lane's item i, over the per-chunk counts
+// of a condition's n chunks (items are numbered in chunk order).  Tiles of 512
+// counts, 8 per lane: a wave scan gives the lanes' offsets, a binary search
+// over the lanes the lane, and its 8 counts the chunk.  Called by a whole wave;
+// lanes without an item pass want = false.
+__device__ __forceinline__ void wave_locate(const int32_t* counts, int n, int64_t i, bool want, int& chunk, int& place) {
+    constexpr int E = 8;
     const int lane = lane_id();
-    const int cid = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (cid >= w.nChunks) return;
-    const Chunk me = w.chunks[cid];
-    const CondParams& cp = w.conds[me.cond];
-    if (!cp.active) return;
-    const PopPlan pl = w.plans[me.cond];
-    const int64_t n = pl.holes < pl.surplus ? pl.holes : pl.surplus;
-    const int64_t* hoff = w.holeOff + cp.chunkBegin;
-    const int64_t* soff = w.surOff + cp.chunkBegin;
-    const int64_t stride = (int64_t)cp.nChunks * kWave;
-    for (int64_t i = (int64_t)me.local * kWave + lane; i < n; i += stride) {
-        const int64_t th = owner_of(hoff, cp.nChunks, i);
-        const Chunk& hc = w.chunks[cp.chunkBegin + th];
-        const int64_t dst = w.holeList[hc.first + (i - hoff[th])];
-        const int64_t ts = owner_of(soff, cp.nChunks, i);
-        const Chunk& sc = w.chunks[cp.chunkBegin + ts];
-        const int64_t src = sc.region + (i - soff[ts]);
-        rec_put(s, dst, rec_get(s, src));
-        s.alive[src] = 0;
-        s.alive[dst] = 1;
-    }
-}
-
-// Holes S..H-1 get clones of uniformly drawn alive main electrons.
-template <typename V>
-__global__ __launch_bounds__(kBlock) void k_clone(DevState<V> s, DevWork w) {
-    const int lane = lane_id();
-    const int cid = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (cid >= w.nChunks) return;
-    const Chunk me = w.chunks[cid];
-    const CondParams& cp = w.conds[me.cond];
-    if (!cp.active) return;
-    const PopPlan pl = w.plans[me.cond];
-    if (pl.holes <= pl.surplus) return;
-    const int64_t* hoff = w.holeOff + cp.chunkBegin;
-    const int64_t stride = (int64_t)cp.nChunks * kWave;
-    double growth = 0;
-    uint32_t status = 0;
-    for (int64_t i = pl.surplus + (int64_t)me.local * kWave + lane; i < pl.holes; i += stride) {
-        const int64_t th = owner_of(hoff, cp.nChunks, i);
-        const Chunk& hc = w.chunks[cp.chunkBegin + th];
-        const int64_t dst = w.holeList[hc.first + (i - hoff[th])];
-        // uniform alive source by rejection over the main slots (BoltzmannMC.C:1368-1371);
-        // draw k of hole i: counter {i, k >> 16, interval, clone | (k & 0xffff)},
-        // so no two of the 2^20 draws share a counter (i < 2^32)
-        int64_t src = -1;
-        for (uint32_t k = 0; k < (1u << 20); ++k) {
-            double u = u53(cp.seed, (uint64_t)(uint32_t)i | ((uint64_t)(k >> 16) << 32), (uint32_t)cp.syncIndex,
-                           P_CLONE, k & 0xffffu);
-            int64_t cand = (int64_t)fmin(floor(u * (double)cp.nMain), (double)(cp.nMain - 1));
-            if (s.alive[cp.base + cand] == 1) { src = cp.base + cand; break; }
+    int64_t running = 0;
+    chunk = 0;
+    place = 0;
+    for (int base = 0; base < n && __ballot(want); base += E * kWave) {
+        int v[E], t = 0;
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int j = base + lane * E + k;
+            v[k] = j < n ? counts[j] : 0;
+            t += v[k];
         }
-        if (src < 0) { status |= ST_POPCTL; continue; }
-        Rec<V> q = rec_get(s, src);
-        growth += rec_energy(q.a);
-        uint32_t wds[4];
-        philox_call(cp.seed ^ 0x5851F42D4C957F2Dull, draw_part(q).stream, (uint32_t)dst, P_CLONE,
-                    (uint32_t)(cp.syncIndex & 0xffffu), wds);
-        draw_part(q).stream = ((uint64_t)wds[1] << 32) | wds[0];
-        draw_part(q).event = 0;
-        rec_put(s, dst, q);
-        s.alive[dst] = 2;  // alive, but not a clone source in this pass (BoltzmannMC.C:1374)
-    }
-    const uint32_t st = wave_or(status);
-    const double g = wave_sum(growth);
-    if (lane == 0) {
-        if (st) atomicOr(&w.status[me.cond], st);
-        w.tailC[(size_t)cid * CT_SIZE + CT_GROWTH] += g;
+        const int first = wave_exclusive_scan(t);
+        const int total = __shfl(first + t, kWave - 1, kWave);
+        const bool here = want && i < running + total;
+        int r = here ? (int)(i - running) : 0;
+        int lo = 0;  // largest lane whose offset is at most r
+#pragma unroll
+        for (int step = kWave / 2; step > 0; step >>= 1)
+            if (__shfl(first, lo + step, kWave) <= r) lo += step;
+        r -= __shfl(first, lo, kWave);
+        bool found = false;
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int m = __shfl(v[k], lo, kWave);
+            if (here && !found) {
+                if (r < m) { chunk = base + lo * E + k; place = r; found = true; }
+                else r -= m;
+            }
+        }
+        want = want && !here;
+        running += total;
     }
 }
 
-// ----------------------------------------------------------------- sample
-// Ensemble sums of one sampling instant (calculateMeanDataForSwarmParams,
-// BoltzmannMC.C:1410-1482) in FP64, per chunk: eps, r, v, r r^T, r v^T,
-// count, max eps.
+// Item i of a condition's holes or surplus newborns: its chunk and place.
+__device__ __forceinline__ void locate(const CondParams& cp, const int32_t* countC, const int64_t* offC, int64_t i,
+                                       bool want, int& chunk, int& place) {
+    if (cp.nChunks <= kPairsDirect) {
+        wave_locate(countC + cp.chunkBegin, cp.nChunks, i, want, chunk, place);
+    } else {
+        const int64_t* off = offC + cp.chunkBegin;
+        chunk = want ? (int)owner_of(off, cp.nChunks, i) : 0;
+        place = want ? (int)(i - off[chunk]) : 0;
+    }
+}
+
+// Index, over a condition's holes in chunk order, of the hole at main slot
+// `slot` (the same in every lane).  Called by a whole wave.
+__device__ int64_t hole_index(const DevWork& w, const CondParams& cp, int64_t slot) {
+    // chunk sizes differ by at most one, the larger ones first
+    const int64_t at = slot - cp.base, each = cp.nMain / cp.nChunks, more = cp.nMain % cp.nChunks;
+    const int64_t big = more * (each + 1);
+    const int j = (int)(at < big ? at / (each + 1) : more + (at - big) / each);
+    const int lane = lane_id();
+    const int64_t first = w.chunks[cp.chunkBegin + j].first;
+    int place = 0;
+    for (int k = lane; k < w.holesC[cp.chunkBegin + j]; k += kWave)
+        if ((int64_t)w.holeList[first + k] == slot) place = k;
+    uint32_t n = (uint32_t)place;  // one lane found it
+    if (cp.nChunks <= kPairsDirect) {
+        for (int k = lane; k < j; k += kWave) n += (uint32_t)w.holesC[cp.chunkBegin + k];
+        return wave_sum_u(n);
+    }
+    return w.holeOff[cp.chunkBegin + j] + wave_sum_u(n);
+}
+
+// Sums over the wave of 26 values per lane, each in the order of a butterfly
+// (wave_sum), transposed: a step halves the values a lane holds, so 32
+// shuffles do what 26 butterflies need 156 for.  Lane l gets the sum of value
+// wave_sums_field(l).
+__device__ __forceinline__ int wave_sums_field(int lane) {
+    return ((lane >> 5) & 1) * 16 + ((lane >> 4) & 1) * 8 + ((lane >> 3) & 1) * 4 + ((lane >> 2) & 1) * 2 + ((lane >> 1) & 1);
+}
+__device__ __forceinline__ double wave_sums(const double (&m)[kMomentRecord], int lane) {
+    double a[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const double lo = m[k], hi = k + 16 < kMomentRecord - 1 ? m[k + 16] : 0.0;
+        const bool up = lane & 32;
+        a[k] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, 32, kWave);
+    }
+#pragma unroll
+    for (int o = 16; o > 1; o >>= 1) {
+        const bool up = lane & o;
+#pragma unroll
+        for (int k = 0; k < o / 2; ++k) {
+            const double lo = a[k], hi = a[k + o / 2];
+            a[k] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, o, kWave);
+        }
+    }
+    return a[0] + __shfl_xor(a[0], 1, kWave);
+}
+
+// ----------------------------------------------------------------- settle
+// The last part of population control and the ensemble sums of one sampling
+// instant, one wave per chunk.
+//  - Pair i of a condition (the waves of its chunks stride over them): hole i
+//    takes surplus newborn i while there are newborns; the remaining holes get
+//    clones of uniformly drawn electrons (BoltzmannMC.C:1368-1371).
+//  - FP64 sums (calculateMeanDataForSwarmParams, BoltzmannMC.C:1410-1482) of
+//    the electrons the chunk holds and of those its wave put into holes: eps,
+//    r, v, r r^T, r v^T, count, max eps.
+// Both in one kernel, so that neither waits for the other: a slot filled here
+// is flagged 2 or 3, by the interval's parity, and the wave that owns the slot
+// neither reads its record nor changes its flag; flags of the interval before
+// become 1.  (With a flag of 1 the flight kernel need store none for an
+// electron that survives its interval: 23 us of it on the 64-condition scan.)
+// On the 64-condition scan the record reads bound it (64 bytes of each
+// electron at the card's copy rate); one condition of 1e4 electrons is bound by
+// the chain of loads.
 template <typename V>
-__global__ __launch_bounds__(kBlock) void k_sample(DevState<V> s, DevWork w) {
+__global__ __launch_bounds__(kBlock) void k_settle(DevState<V> s, DevWork w) {
     const int lane = lane_id();
     const int cid = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
     if (cid >= w.nChunks) return;
-    const Chunk ch = w.chunks[cid];
-    if (!w.conds[ch.cond].active) return;
+    const Chunk me = w.chunks[cid];
+    const CondParams& cp = w.conds[me.cond];
+    if (!cp.active) return;
+    const uint8_t filled = (uint8_t)(2 + (cp.syncIndex & 1));
     double m[kMomentRecord];
+#pragma unroll
     for (int k = 0; k < kMomentRecord; ++k) m[k] = 0;
     auto add = [&](const RecA<V>& q) {
         const double r[3] = {q.x, q.y, q.z};
@@ -1158,30 +1331,93 @@ __global__ __launch_bounds__(kBlock) void k_sample(DevState<V> s, DevWork w) {
         m[25] += 1;
         m[26] = fmax(m[26], e);
     };
-    // two records per lane in flight; each lane still adds its records in
-    // slot order.  The clone marks (alive flag 2) of this interval's
-    // population control end here, read with the records: the flight kernel
-    // then stores no flag for an electron that survives its interval (a
-    // one-byte store per electron that shared HBM sectors with its
-    // neighbours: flight kernel 0.917 -> 0.894 ms per interval on the
-    // 64-condition scan, this kernel 1 us slower)
+
+    const CondPop pop = pop_total(w, me.cond);
+    const bool removed = pop.surplus > pop.holes;  // then as many newborns as holes are left
+    const int64_t H = removed ? pop.holesAfter : pop.holes, S = removed ? pop.holesAfter : pop.surplus;
+    const int64_t stride = (int64_t)cp.nChunks * kWave;
+    double growth = 0;
+    uint32_t status = 0;
+    for (int64_t i0 = (int64_t)me.local * kWave; i0 < H; i0 += stride) {
+        const int64_t i = i0 + lane;
+        const bool want = i < H, move = i < S;
+        int hc, hp, sc, sp;
+        locate(cp, w.holesC, w.holeOff, i, want, hc, hp);
+        locate(cp, w.surplusC, w.surOff, i, move, sc, sp);
+        int64_t src = -1;
+        if (move) src = w.chunks[cp.chunkBegin + sc].region + sp;
+        // uniform alive source by rejection over the main slots (BoltzmannMC.C:1368-1371);
+        // draw k of hole i: counter {i, k >> 16, interval, clone | (k & 0xffff)},
+        // so no two of the 2^20 draws share a counter (i < 2^32)
+        bool seek = want && !move;
+        for (uint32_t k = 0; k < (1u << 20) && __ballot(seek); ++k) {
+            int64_t cand = 0;
+            bool hole = false;
+            if (seek) {
+                const double u = u53(cp.seed, (uint64_t)(uint32_t)i | ((uint64_t)(k >> 16) << 32),
+                                     (uint32_t)cp.syncIndex, P_CLONE, k & 0xffffu);
+                cand = cp.base + (int64_t)fmin(floor(u * (double)cp.nMain), (double)(cp.nMain - 1));
+                const uint8_t a = s.alive[cand];
+                hole = a == 0 || a == filled;
+                if (!hole) { src = cand; seek = false; }
+            }
+            // a hole is a source where a newborn takes it; its record is read
+            // where the newborn is
+            for (uint64_t hm = S > 0 ? __ballot(hole) : 0; hm; hm &= hm - 1) {
+                const int l = __ffsll((unsigned long long)hm) - 1;
+                const int64_t j = hole_index(w, cp, __shfl(cand, l, kWave));
+                if (j >= S) continue;
+                int nc, np;
+                locate(cp, w.surplusC, w.surOff, j, lane == l, nc, np);
+                if (lane == l) { src = w.chunks[cp.chunkBegin + nc].region + np; seek = false; }
+            }
+        }
+        if (!want) continue;
+        if (src < 0) { status |= ST_POPCTL; continue; }
+        const int64_t dst = w.holeList[w.chunks[cp.chunkBegin + hc].first + hp];
+        Rec<V> q = rec_get(s, src);
+        if (move) {
+            s.alive[src] = 0;
+        } else {
+            growth += rec_energy(q.a);
+            uint32_t wds[4];
+            philox_call(cp.seed ^ 0x5851F42D4C957F2Dull, draw_part(q).stream, (uint32_t)dst, P_CLONE,
+                        (uint32_t)(cp.syncIndex & 0xffffu), wds);
+            draw_part(q).stream = ((uint64_t)wds[1] << 32) | wds[0];
+            draw_part(q).event = 0;
+        }
+        rec_put(s, dst, q);
+        s.alive[dst] = filled;
+        add(q.a);
+    }
+
+    // two records per lane in flight; each lane adds its records in slot order
+    auto own = [&](const RecA<V>& q, uint8_t a, int64_t slot) {
+        if (a == 0 || a == filled) return;  // a hole before the pairs
+        add(q);
+        if (a != 1) s.alive[slot] = 1;
+    };
     int64_t k = lane;
-    for (; k + kWave < ch.count; k += 2 * kWave) {
-        const RecA<V> q0 = s.ra[ch.first + k], q1 = s.ra[ch.first + k + kWave];
-        const uint8_t a0 = s.alive[ch.first + k], a1 = s.alive[ch.first + k + kWave];
-        add(q0);
-        add(q1);
-        if (a0 == 2) s.alive[ch.first + k] = 1;
-        if (a1 == 2) s.alive[ch.first + k + kWave] = 1;
+    for (; k + kWave < me.count; k += 2 * kWave) {
+        const RecA<V> q0 = s.ra[me.first + k], q1 = s.ra[me.first + k + kWave];
+        const uint8_t a0 = s.alive[me.first + k], a1 = s.alive[me.first + k + kWave];
+        own(q0, a0, me.first + k);
+        own(q1, a1, me.first + k + kWave);
     }
-    if (k < ch.count) {
-        add(s.ra[ch.first + k]);
-        if (s.alive[ch.first + k] == 2) s.alive[ch.first + k] = 1;
+    if (k < me.count) own(s.ra[me.first + k], s.alive[me.first + k], me.first + k);
+    const double mx = wave_max(m[26]);
+    m[26] = 0;
+    const double sum = wave_sums(m, lane);
+    const uint32_t st = wave_or(status);
+    const double g = H > S ? wave_sum(growth) : 0.0;
+    double* out = w.momC + (size_t)cid * kMomentRecord;
+    const int f = wave_sums_field(lane);
+    if ((lane & 1) == 0 && f < kMomentRecord - 1) out[f] = sum;
+    if (lane == 1) out[kMomentRecord - 1] = mx;
+    if (lane == 0) {
+        if (st) atomicOr(&w.status[me.cond], st);
+        if (g != 0) w.tailC[(size_t)cid * CT_SIZE + CT_GROWTH] += g;
     }
-    for (int k = 0; k < kMomentRecord - 1; ++k) m[k] = wave_sum(m[k]);
-    m[26] = wave_max(m[26]);
-    if (lane == 0)
-        for (int k = 0; k < kMomentRecord; ++k) w.momC[(size_t)cid * kMomentRecord + k] = m[k];
 }
 
 // Histograms of one sampling instant (getTimeDependDistributions,
@@ -1250,53 +1486,53 @@ __global__ __launch_bounds__(kBlock) void k_hist(DevState<V> s, const SlotRange*
 
 // ----------------------------------------------------------------- finish
 // summary[c] = [ event record (3P + 8) | moment sums (kMomentRecord) | plan (8) ]
-// Chunk records are summed in a fixed order: thread t adds chunks t, t+256,
-// ... in order, the wave adds its lanes by butterflies, and thread f adds the
-// four waves in order.  The integer accumulators are converted and cleared
-// for the next interval.  Block 0 resets the flight-kernel work queues.
+// Chunk records are summed in a fixed order: thread (r, f) of a block adds
+// field f of records r, r + kFinishRows, ... in order (neighbouring threads
+// read neighbouring fields), then thread f adds the rows.  The integer
+// accumulators are converted and cleared for the next interval, and block 0
+// resets the flight-kernel work queues.
 constexpr int kFinishFields = CT_SIZE + kMomentRecord;
-// Fixed-order sums (maxima for the two maximum fields) over the records
-// [first, first + n) of a chunk-tail array and a moment array, by one
-// 256-thread block: each thread takes records threadIdx.x, + 256, ..., the
-// waves reduce by shuffles and thread f < kFinishFields adds the four wave
-// results of field f in wave order; the result is valid in those threads.
+constexpr int kFinishBlock = 1024;
+constexpr int kFinishRows = kFinishBlock / (kFinishFields + 1);
+// Sums (maxima for the two maximum fields) over the records [first, first + n)
+// of a chunk-tail array and a moment array by one block; the result is valid
+// in threads f < kFinishFields.  One thread per record with every field in
+// registers and 35 wave reductions took 12.6 us for the 40 records of one
+// condition of 1e4 electrons, this 5.2 us.
 __device__ double finish_reduce(const double* tsrc, const double* msrc, size_t first, int n,
-                                double (*red)[256 / kWave]) {
-    double acc[kFinishFields];
-#pragma unroll
-    for (int f = 0; f < kFinishFields; ++f) acc[f] = 0;
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
-        const size_t j = first + k;
-        const double* t = tsrc + j * CT_SIZE;
-        const double* m = msrc + j * kMomentRecord;
-#pragma unroll
-        for (int f = 0; f < CT_SIZE; ++f) acc[f] = f == CT_MAXE ? fmax(acc[f], t[f]) : acc[f] + t[f];
-#pragma unroll
-        for (int f = 0; f < kMomentRecord; ++f)
-            acc[CT_SIZE + f] = f == kMomentRecord - 1 ? fmax(acc[CT_SIZE + f], m[f]) : acc[CT_SIZE + f] + m[f];
-    }
-    const int lane = lane_id(), wid = threadIdx.x / kWave;
-#pragma unroll
-    for (int f = 0; f < kFinishFields; ++f) {
-        const bool isMax = f == CT_MAXE || f == kFinishFields - 1;
-        const double v = isMax ? wave_max(acc[f]) : wave_sum(acc[f]);
-        if (lane == 0) red[f][wid] = v;
+                                double (*red)[kFinishFields + 1]) {
+    const int row = threadIdx.x / (kFinishFields + 1), f = threadIdx.x % (kFinishFields + 1);
+    const bool isMax = f == CT_MAXE || f == kFinishFields - 1;
+    if (row < kFinishRows && f < kFinishFields) {
+        const double* src = f < CT_SIZE ? tsrc + first * CT_SIZE + f : msrc + first * kMomentRecord + (f - CT_SIZE);
+        const int each = f < CT_SIZE ? CT_SIZE : kMomentRecord;
+        double acc = 0;
+#pragma unroll 8
+        for (int k = row; k < n; k += kFinishRows) {
+            const double v = src[(size_t)k * each];
+            acc = isMax ? fmax(acc, v) : acc + v;
+        }
+        red[row][f] = acc;
     }
     __syncthreads();
     double tot = 0;
     if (threadIdx.x < kFinishFields) {
-        const int f = threadIdx.x;
-        const bool isMax = f == CT_MAXE || f == kFinishFields - 1;
-        tot = red[f][0];
-        for (int i = 1; i < 256 / kWave; ++i) tot = isMax ? fmax(tot, red[f][i]) : tot + red[f][i];
+        const bool top = threadIdx.x == CT_MAXE || threadIdx.x == kFinishFields - 1;
+        double part[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int r = 0; r < kFinishRows; ++r) {
+            const double v = red[r][threadIdx.x];
+            part[r & 3] = top ? fmax(part[r & 3], v) : part[r & 3] + v;
+        }
+        tot = top ? fmax(fmax(part[0], part[1]), fmax(part[2], part[3])) : (part[0] + part[1]) + (part[2] + part[3]);
     }
     return tot;
 }
 
 // First pass for conditions with many work units: group g's sums, in the
 // record layout of the chunk tails and moments.
-__global__ __launch_bounds__(256) void k_finish_group(DevWork w) {
-    __shared__ double red[kFinishFields][256 / kWave];
+__global__ __launch_bounds__(kFinishBlock) void k_finish_group(DevWork w) {
+    __shared__ double red[kFinishRows][kFinishFields + 1];
     const int g = blockIdx.x;
     if (!w.conds[w.groupCond[g]].active) return;
     const double tot = finish_reduce(w.tailC, w.momC, (size_t)w.groupFirst[g], w.groupCount[g], red);
@@ -1307,8 +1543,8 @@ __global__ __launch_bounds__(256) void k_finish_group(DevWork w) {
     }
 }
 
-__global__ __launch_bounds__(256) void k_finish(DevWork w, int P) {
-    __shared__ double red[kFinishFields][256 / kWave];
+__global__ __launch_bounds__(kFinishBlock) void k_finish(DevWork w, int P) {
+    __shared__ double red[kFinishRows][kFinishFields + 1];
     const int c = blockIdx.x;
     if (c == 0 && threadIdx.x < 8) w.queue[threadIdx.x] = 0;
     const CondParams cp = w.conds[c];
@@ -1333,12 +1569,14 @@ __global__ __launch_bounds__(256) void k_finish(DevWork w, int P) {
         w.accLoss[i] = 0;
     }
     if (threadIdx.x == 0) {
-        const PopPlan pl = w.plans[c];
+        const CondPop pop = pop_total(w, c);
+        const PopPlan pl = plan_of(pop, cp);
         double* tail = out + R + kMomentRecord;
         tail[0] = (double)pl.holes; tail[1] = (double)pl.surplus; tail[2] = (double)pl.alive;
-        tail[3] = (double)pl.remove; tail[4] = (double)pl.marks; tail[5] = (double)pl.thrIndex;
+        tail[3] = (double)pl.remove; tail[4] = (double)pop.marks; tail[5] = 0;
         tail[6] = (double)w.status[c];
         tail[7] = 0;
+        for (int k = 0; k < kPopCopies; ++k) w.pop[(size_t)k * w.popStride + c] = CondPop{};
     }
 }
 
@@ -1630,33 +1868,22 @@ hipError_t launch_flights(const DevState<V>& s, const DevWork& w, const DevProce
 template <typename V>
 hipError_t launch_popctl(const DevState<V>& s, const DevWork& w, hipStream_t st) {
     const dim3 g(chunk_grid(w.nChunks)), b(kBlock);
-    timer_start(K_PLAN, st);
-    hipLaunchKernelGGL(k_plan, dim3(w.nCond), dim3(1024), 0, st, w);
-    timer_stop(K_PLAN, st);
     timer_start(K_MARKS, st);
     hipLaunchKernelGGL(k_marks, g, b, 0, st, s.alive, w);
-    hipLaunchKernelGGL(k_plan_marks, dim3(w.nCond), dim3(1024), 0, st, w);
+    if (w.planMarks) hipLaunchKernelGGL(k_plan_marks, dim3(w.nCond), dim3(1024), 0, st, w);
     timer_stop(K_MARKS, st);
     timer_start(K_APPLY, st);
     hipLaunchKernelGGL(k_apply_marks<V>, g, b, 0, st, s, w);
+    if (w.planPairs) hipLaunchKernelGGL(k_plan_pairs, dim3(w.nCond), dim3(1024), 0, st, w);
     timer_stop(K_APPLY, st);
-    timer_start(K_PAIRS, st);
-    hipLaunchKernelGGL(k_plan_pairs, dim3(w.nCond), dim3(1024), 0, st, w);
-    timer_stop(K_PAIRS, st);
-    timer_start(K_MOVE, st);
-    hipLaunchKernelGGL(k_move<V>, g, b, 0, st, s, w);
-    timer_stop(K_MOVE, st);
-    timer_start(K_CLONE, st);
-    hipLaunchKernelGGL(k_clone<V>, g, b, 0, st, s, w);
-    timer_stop(K_CLONE, st);
     return hipGetLastError();
 }
 
 template <typename V>
-hipError_t launch_sample(const DevState<V>& s, const DevWork& w, hipStream_t st) {
-    timer_start(K_SAMPLE, st);
-    hipLaunchKernelGGL(k_sample<V>, dim3(chunk_grid(w.nChunks)), dim3(kBlock), 0, st, s, w);
-    timer_stop(K_SAMPLE, st);
+hipError_t launch_settle(const DevState<V>& s, const DevWork& w, hipStream_t st) {
+    timer_start(K_SETTLE, st);
+    hipLaunchKernelGGL(k_settle<V>, dim3(chunk_grid(w.nChunks)), dim3(kBlock), 0, st, s, w);
+    timer_stop(K_SETTLE, st);
     return hipGetLastError();
 }
 
@@ -1673,8 +1900,8 @@ hipError_t launch_hist(const DevState<V>& s, const DevHist& h, hipStream_t st) {
 
 hipError_t launch_finish(const DevWork& w, int P, hipStream_t st) {
     timer_start(K_REDUCE, st);
-    if (w.nGroups) hipLaunchKernelGGL(k_finish_group, dim3(w.nGroups), dim3(256), 0, st, w);
-    hipLaunchKernelGGL(k_finish, dim3(w.nCond), dim3(256), 0, st, w, P);
+    if (w.nGroups) hipLaunchKernelGGL(k_finish_group, dim3(w.nGroups), dim3(kFinishBlock), 0, st, w);
+    hipLaunchKernelGGL(k_finish, dim3(w.nCond), dim3(kFinishBlock), 0, st, w, P);
     timer_stop(K_REDUCE, st);
     return hipGetLastError();
 }
@@ -1710,7 +1937,7 @@ hipError_t launch_op_philox(int64_t n, const uint32_t* ctr, const uint32_t* key,
     template hipError_t launch_flights<V>(const DevState<V>&, const DevWork&, const DevProcesses&, const V*,  \
                                           const DevHist&, const FlightLists&, hipStream_t);                   \
     template hipError_t launch_popctl<V>(const DevState<V>&, const DevWork&, hipStream_t);                    \
-    template hipError_t launch_sample<V>(const DevState<V>&, const DevWork&, hipStream_t);                    \
+    template hipError_t launch_settle<V>(const DevState<V>&, const DevWork&, hipStream_t);                    \
     template hipError_t launch_hist<V>(const DevState<V>&, const DevHist&, hipStream_t);                     \
     template int flight_blocks_per_cu<V>(int, bool, int, const DevHist&);                                                \
     template hipError_t launch_tables<V>(const DevTableSrc&, double, double, int, V*, double*, double*,        \

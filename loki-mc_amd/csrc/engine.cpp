@@ -558,8 +558,8 @@ public:
         HIP_TRY(hipMemsetAsync(accCount.p, 0, (size_t)n * P * 8, stream));
         HIP_TRY(hipMemsetAsync(accGain.p, 0, (size_t)n * P * 8, stream));
         HIP_TRY(hipMemsetAsync(accLoss.p, 0, (size_t)n * P * 8, stream));
-        HIP_TRY(queue.alloc(8));
-        HIP_TRY(hipMemsetAsync(queue.p, 0, 8 * sizeof(uint32_t), stream));
+        HIP_TRY(queue.alloc(kFlightClasses * kXcds * kQueueStride));
+        HIP_TRY(hipMemsetAsync(queue.p, 0, queue.n * sizeof(uint32_t), stream));
         HIP_TRY(plans.alloc(n));
         HIP_TRY(status.alloc(n));
         HIP_TRY(hipMemsetAsync(status.p, 0, n * sizeof(uint32_t), stream));
@@ -837,18 +837,29 @@ public:
             // processing order does not change any result (flight kernel per
             // interval on the 64-condition scan: 0.896 ms ordered by size,
             // 0.890 ms by expected work)
-            std::stable_sort(hlist.begin() + begin, hlist.end(), [&](int32_t a, int32_t b) {
-                return hchunks[a].count * cs[hchunks[a].cond].workPerElectron >
-                       hchunks[b].count * cs[hchunks[b].cond].workPerElectron;
-            });
-            const int32_t count = (int32_t)(hlist.size() - begin);
-            fl.list[fc] = flist.p + begin;
-            fl.count[fc] = count;
-            if (count) {
-                const int64_t waves = (int64_t)flight_blocks_per_cu<V>(fc, thermal, P, dh) * cus;
-                const int64_t need = (count + kBlock / kWave - 1) / (kBlock / kWave);
-                fl.grid[fc] = (int32_t)std::max<int64_t>(1, std::min<int64_t>(need, waves));
+            auto work_of = [&](int32_t k) { return hchunks[k].count * cs[hchunks[k].cond].workPerElectron; };
+            std::stable_sort(hlist.begin() + begin, hlist.end(),
+                             [&](int32_t a, int32_t b) { return work_of(a) > work_of(b); });
+            const int64_t count = (int64_t)(hlist.size() - begin);
+            if (count == 0) continue;
+            FlightList& l = fl.cls[fc];
+            l.list = flist.p + begin;
+            const int64_t waves = (int64_t)flight_blocks_per_cu<V>(fc, thermal, P, dh) * cus * (kBlock / kWave);
+            l.oneShot = count <= waves;
+            // parts of equal chunk count (one shot) or of equal expected work
+            double total = 0, sum = 0;
+            for (int64_t k = 0; k < count; ++k) total += work_of(hlist[begin + k]);
+            int x = 0;
+            for (int64_t k = 0; k < count; ++k) {
+                const bool next = l.oneShot ? k * kXcds >= x * count : sum * kXcds >= x * total;
+                if (next && x < kXcds) l.part[x++] = (int32_t)k;
+                sum += work_of(hlist[begin + k]);
             }
+            while (x <= kXcds) l.part[x++] = (int32_t)count;
+            int64_t longest = 0;
+            for (x = 0; x < kXcds; ++x) longest = std::max<int64_t>(longest, l.part[x + 1] - l.part[x]);
+            const int64_t perBlock = kBlock / kWave;
+            fl.grid[fc] = (int32_t)(l.oneShot ? kXcds * ((longest + perBlock - 1) / perBlock) : waves / perBlock);
         }
         if (!hlist.empty())
             HIP_TRY(hipMemcpyAsync(flist.p, hlist.data(), hlist.size() * sizeof(int32_t), hipMemcpyHostToDevice, stream));

@@ -117,7 +117,7 @@ struct DevWork {
     long long* accLoss;           // [n_cond * P]
     PopPlan* plans;               // [n_cond]
     uint32_t* status;             // [n_cond]
-    uint32_t* queue;              // [8] work-queue counters of the flight kernels
+    uint32_t* queue;              // [kFlightClasses * kXcds * kQueueStride] work-queue counters of the flight kernels
     double* summary;              // [n_cond * summarySize]
     int summarySize;
     int recSize;                  // 3P + 8
@@ -178,11 +178,17 @@ struct DevHist {
 };
 
 // Flight-kernel work lists, one per field case (or FLIGHT_DC_ANY): chunk ids
-// in processing order.
+// in processing order, in one contiguous part per XCD.
+constexpr int kXcds = 8;
+constexpr int kQueueStride = 32;   // work-queue counters 128 bytes apart
+struct FlightList {
+    const int32_t* list;
+    int32_t part[kXcds + 1];       // part x is list[part[x], part[x + 1])
+    int32_t oneShot;               // the grid has a wave for every chunk
+};
 struct FlightLists {
-    const int32_t* list[kFlightClasses];
-    int32_t count[kFlightClasses];
-    int32_t grid[kFlightClasses];  // persistent blocks per launch
+    FlightList cls[kFlightClasses];
+    int32_t grid[kFlightClasses];  // blocks per launch (0: no chunk)
 };
 
 // Sources of the collision tables (interpolateCrossSections,

@@ -770,12 +770,19 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
 // fit the LDS) spilled 33-41 VGPRs and ran at 1.062 ms.
 template <typename V, int FC> constexpr int flight_waves_per_eu() { return sizeof(V) == 8 ? 2 : 1; }
 
-// Persistent flight kernel of one field case: every wave takes chunks from
-// the list through an atomic counter until the list is exhausted.
+// Flight kernel of one field case.  The work list has one part per XCD
+// (kXcds contiguous parts of about equal work; blocks go to the XCDs in turn):
+// chunks of one condition then run on one XCD, or on neighbouring ones, at about
+// the same time, and its tables and cylindrical histograms stay in that XCD's
+// L2.  Where the grid has a wave for every chunk a wave takes the chunk of its
+// place; otherwise waves take chunks of their XCD's part through an atomic
+// counter, then of the other parts, until the list is exhausted.  (Flight kernel per
+// interval, one queue for all XCDs against this: 8 conditions of 1e5 with EADF
+// and EVDF 146 -> 126 us, one condition of 9.5e5 in FP64 155 -> 148 us, 24 AC
+// conditions of 2e5 557 -> 523 us; no difference for the 64-condition scan.)
 template <typename V, int FC, bool THERMAL, int HIST>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_waves_per_eu<V, FC>()))) void k_advance(DevState<V> s, DevWork w, DevProcesses pr, const V* tables,
-                                                    DevHist h, const int32_t* list, int32_t nList,
-                                                    uint32_t* queue) {
+                                                    DevHist h, FlightList fl, uint32_t* queue) {
     extern __shared__ unsigned char smem[];
     constexpr int kRingWave = ring_segs<V>() * rec_pieces<V>() * kRingSeg;  // 16-byte pieces per wave
     __shared__ uint4 rings[kWavesPerBlock * kRingWave];
@@ -791,12 +798,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_w
     unsigned long long* cnt =
         (unsigned long long*)(smem + (size_t)pr.P * sizeof(ProcRec) + (size_t)wid * flight_wave_lds<V>(pr.P, h.histLds));
     lds_uint4* ring = (lds_uint4*)(rings + wid * kRingWave);
-    while (true) {
-        uint32_t item = 0;
-        if (lane_id() == 0) item = atomicAdd(queue, 1u);
-        item = (uint32_t)__builtin_amdgcn_readfirstlane((int)__shfl((int)item, 0, kWave));
-        if (item >= (uint32_t)nList) break;
-        advance_chunk<V, FC, THERMAL, HIST>(s, w, prl, tables, h, list[item], cnt, ring);
+    const int xcd = blockIdx.x % kXcds;
+    int x = xcd;
+    while (true) {  // one call of advance_chunk: two would be inlined twice (174 VGPRs)
+        uint32_t item = (blockIdx.x / kXcds) * kWavesPerBlock + wid;
+        if (!fl.oneShot && lane_id() == 0) item = atomicAdd(&queue[x * kQueueStride], 1u);
+        item = (uint32_t)__builtin_amdgcn_readfirstlane((int)item) + (uint32_t)fl.part[x];
+        if (item >= (uint32_t)fl.part[x + 1]) {
+            x = x + 1 < kXcds ? x + 1 : 0;
+            if (fl.oneShot || x == xcd) break;
+            continue;
+        }
+        advance_chunk<V, FC, THERMAL, HIST>(s, w, prl, tables, h, fl.list[item], cnt, ring);
+        if (fl.oneShot) break;
     }
 }
 
@@ -1546,7 +1560,8 @@ __global__ __launch_bounds__(kFinishBlock) void k_finish_group(DevWork w) {
 __global__ __launch_bounds__(kFinishBlock) void k_finish(DevWork w, int P) {
     __shared__ double red[kFinishRows][kFinishFields + 1];
     const int c = blockIdx.x;
-    if (c == 0 && threadIdx.x < 8) w.queue[threadIdx.x] = 0;
+    if (c == 0)
+        for (int k = threadIdx.x; k < kFlightClasses * kXcds; k += blockDim.x) w.queue[k * kQueueStride] = 0;
     const CondParams cp = w.conds[c];
     if (!cp.active) return;
     double* out = w.summary + (size_t)c * w.summarySize;
@@ -1805,8 +1820,8 @@ static void launch_advance_hist(const DevState<V>& s, const DevWork& w, const De
                                 const DevHist& h, const FlightLists& fl, hipStream_t st) {
     dim3 g(fl.grid[FC]), b(kBlock);
     const size_t lds = flight_lds<V>(pr.P, h.histLds);
-    hipLaunchKernelGGL((k_advance<V, FC, TH, HIST>), g, b, lds, st, s, w, pr, tables, h, fl.list[FC], fl.count[FC],
-                       w.queue + FC);
+    hipLaunchKernelGGL((k_advance<V, FC, TH, HIST>), g, b, lds, st, s, w, pr, tables, h, fl.cls[FC],
+                       w.queue + FC * kXcds * kQueueStride);
 }
 
 template <typename V, int FC, bool TH>
@@ -1822,7 +1837,7 @@ static void launch_advance_th(const DevState<V>& s, const DevWork& w, const DevP
 template <typename V, int FC>
 static void launch_advance_case(const DevState<V>& s, const DevWork& w, const DevProcesses& pr, const V* tables,
                                 const DevHist& h, const FlightLists& fl, hipStream_t st) {
-    if (fl.count[FC] == 0) return;
+    if (fl.grid[FC] == 0) return;
     if (pr.gasTempEffect == 0) launch_advance_th<V, FC, false>(s, w, pr, tables, h, fl, st);
     else launch_advance_th<V, FC, true>(s, w, pr, tables, h, fl, st);
 }

@@ -29,7 +29,15 @@ HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC",
 SOURCES = ["kernels.hip", "tables.cpp", "engine.cpp"]
 # FP32 division and square root of the mixed form without IEEE rounding
 # (a few ulp); FP64 arithmetic is unaffected.
-EXTRA = {"kernels.hip": ["-fno-hip-fp32-correctly-rounded-divide-sqrt"]}
+# No hoisting of machine instructions out of loops: what it hoists out of the
+# flight kernel's step loop are the FP64 literals of log, sin, cos and pow, and
+# the registers to hold them take the FP64 form from 165 VGPRs to 256 with
+# spills, and spill 100-200 SGPRs into VGPR lanes that the loop reads back one by
+# one (v_readlane in the FP64 kernel of the crossed-field scan 408 -> 156).
+# Flight kernel per interval, with it against without: 64-condition scan in
+# FP64 1474 -> 1376 us, one condition of 9.5e5 in FP64 152 -> 145, one of 1e8 in
+# mixed precision with thermal targets 19.25 -> 19.04 ms, mixed scan 877 -> 882 us.
+EXTRA = {"kernels.hip": ["-fno-hip-fp32-correctly-rounded-divide-sqrt", "-mllvm", "-disable-machine-licm"]}
 
 
 def _hipcc():

@@ -66,29 +66,39 @@ __device__ __forceinline__ constexpr int half64(int s) {
     return (s == 5 || s == 7 || s == 2 || s == 4 || s == 9) ? 1 : 0;
 }
 
-// Variates of one event: call 0 cached in w0, one other call in w1.  With a
-// tape (batch operators) the slot values are read from it instead.
+// Variates of one event: call 0 in w0, call 1 in w1, one other call in wx.  With
+// a tape (batch operators) the slot values are read from it instead.  A wave's
+// lanes need a call's words for different reasons (a free time to draw, or a
+// pending one that ends in a collision; one scattering model or another):
+// where nearly every lane needs a call it is drawn once before the lanes part,
+// not in each of the branches, each of which the wave would run in turn.  (Flight
+// kernel per interval, mixed: the 64-condition scan 882 -> 861 us, one condition
+// of 1e4 electrons 49.7 -> 47.2; FP64: four ECR conditions 93 -> 88 us.)
 template <typename V> struct EventRng {
     uint64_t seed, stream;
     uint32_t event;
-    bool have0;
+    bool have0, have1;
     int other;
-    uint32_t w0[4], w1[4];
+    uint32_t w0[4], w1[4], wx[4];
     const double* tape;
     __device__ EventRng(uint64_t sd, uint64_t st, uint32_t ev, const double* tp = nullptr)
-        : seed(sd), stream(st), event(ev), have0(false), other(-1), tape(tp) {}
+        : seed(sd), stream(st), event(ev), have0(false), have1(false), other(-1), tape(tp) {}
     // with call 0 already drawn
     __device__ EventRng(uint64_t sd, uint64_t st, uint32_t ev, const uint32_t c0[4])
-        : seed(sd), stream(st), event(ev), have0(true), other(-1), tape(nullptr) {
+        : seed(sd), stream(st), event(ev), have0(true), have1(false), other(-1), tape(nullptr) {
         w0[0] = c0[0]; w0[1] = c0[1]; w0[2] = c0[2]; w0[3] = c0[3];
     }
     __device__ __forceinline__ void prime0() {
         if (!have0) { philox_call(seed, stream, event, P_EVENT, 0u, w0); have0 = true; }
     }
+    __device__ __forceinline__ void prime1() {
+        if (!have1) { philox_call(seed, stream, event, P_EVENT, 1u, w1); have1 = true; }
+    }
     __device__ __forceinline__ const uint32_t* words(int call) {
         if (call == 0) { prime0(); return w0; }
-        if (other != call) { philox_call(seed, stream, event, P_EVENT, (uint32_t)call, w1); other = call; }
-        return w1;
+        if (call == 1) { prime1(); return w1; }
+        if (other != call) { philox_call(seed, stream, event, P_EVENT, (uint32_t)call, wx); other = call; }
+        return wx;
     }
     __device__ __forceinline__ V u(int s);
 };
@@ -326,29 +336,32 @@ __device__ inline void flight(const CondParams& c, Electron<float>& e, double dt
 }
 
 // --------------------------------------------------------------- samplers
-// AngularScatteringFunctions.h:27-74; `slot` is the variate slot.
+// AngularScatteringFunctions.h:27-74; `slot` is the variate slot.  The variate
+// and the power are taken once for all models.
 template <typename V>
 __device__ __forceinline__ V cos_chi(const DevProcesses& pr, int p, V energy, V energyAfter, EventRng<V>& rng,
                                     int slot) {
-    switch (pr.proc[p].scat) {
-        case 1: return (V)1;  // forward
-        case 2: {             // bornDipole
+    const int scat = pr.proc[p].scat;
+    const V R = rng.u(slot);
+    if (scat == 2 || scat == 3) {  // bornDipole, surendra
+        V r2 = (V)0;
+        if (scat == 2) {
             V loss = (V)pr.proc[p].energyLoss;
             V s = sqrt(energyAfter) + sqrt(energy);
             V ratio = loss / (s * s);
-            V r2 = ratio * ratio;
-            return (V)1 + (V)2 * r2 / ((V)1 - r2) * ((V)1 - pow(r2, -rng.u(slot)));
+            r2 = ratio * ratio;
         }
-        case 3:  // surendra
-            return ((V)2 + energy - (V)2 * pow((V)1 + energy, rng.u(slot))) / energy;
-        case 4: {  // coulombScreen
-            V eps = pr.proc[p].params[0] == 0 ? energy : energyAfter;
-            V sp = (V)pr.proc[p].params[1] / eps;
-            V R = rng.u(slot);
-            return (sp + (V)1 - ((V)2 * sp + (V)1) * R) / (sp + (V)1 - R);
-        }
-        default: return (V)1 - (V)2 * rng.u(slot);  // isotropic
+        const V pw = pow(scat == 2 ? r2 : (V)1 + energy, scat == 2 ? -R : R);
+        if (scat == 2) return (V)1 + (V)2 * r2 / ((V)1 - r2) * ((V)1 - pw);
+        return ((V)2 + energy - (V)2 * pw) / energy;
     }
+    if (scat == 4) {  // coulombScreen
+        V eps = pr.proc[p].params[0] == 0 ? energy : energyAfter;
+        V sp = (V)pr.proc[p].params[1] / eps;
+        return (sp + (V)1 - ((V)2 * sp + (V)1) * R) / (sp + (V)1 - R);
+    }
+    if (scat == 1) return (V)1;  // forward
+    return (V)1 - (V)2 * R;      // isotropic
 }
 
 // sin(chi) of a sampled cos(chi).  A sampler can round past 1: the FP32
@@ -514,11 +527,19 @@ __device__ __forceinline__ int cold_choose(const CondParams& c, const DevProcess
 }
 
 // Thermal channel choice (BoltzmannMC.C:916-1031): target velocity Vt from
-// three normals; -1 for a null collision.
+// three normals; -1 for a null collision.  `gasSum` [I*G] holds the sum over
+// each gas's processes, cumul[R] - cumul[L - 1] as the reference forms it.
+// A gas's row depends on its own relative speed, not on the gases before it, so
+// the sums of four gases are loaded together; the search then runs in the
+// cumulative table of the one gas that was hit.  (Gas by gas in the cumulative
+// table, a null collision of five gases made five dependent round trips to two
+// far apart entries each, in a table of 8 MB instead of 0.2: flight kernel of one
+// condition of 1e8 electrons, 200 processes, 19.0 -> 14.6 ms per interval.)
 template <typename V>
 __device__ __forceinline__ int thermal_choose(const CondParams& c, const DevProcesses& pr, const V* cumul,
-                                              const V* interp, const Electron<V>& e, EventRng<V>& rng, V Vt[3]) {
-    const int P = pr.P, I = c.I;
+                                              const V* interp, const V* gasSum, const Electron<V>& e,
+                                              EventRng<V>& rng, V Vt[3]) {
+    const int P = pr.P, I = c.I, G = pr.G;
     const V step = (V)c.step;
     // MathFunctions::unitNormalRand3 (MathFunctions.C:54-59)
     const V r5 = rng.u(5);
@@ -529,38 +550,64 @@ __device__ __forceinline__ int thermal_choose(const CondParams& c, const DevProc
     V aux1 = sqrt((V)-2 * log_of(r1));
     V vers[3] = {aux1 * c2r, aux1 * s2, sqrt((V)-2 * log_of(r3)) * c4r};
     V randCS = e.nue * r5 / (V)c.N;
-    V prevSum = (V)0;
-    for (int g = 0; g < pr.G; ++g) {
-        if (pr.gasFrac[g] == 0) continue;
-        int L = pr.gasFirst[g], R = pr.gasLast[g];
-        V sd = (V)pr.proc[L].thermalStd;
-        for (int k = 0; k < 3; ++k) Vt[k] = vers[k] * sd;
-        V dx = e.vx - Vt[0], dy = e.vy - Vt[1], dz = e.vz - Vt[2];
-        V rel = sqrt(sqr_norm(dx, dy, dz));
-        V over = (V)0.5 * (V)pr.proc[L].rMass * rel * rel / (V)kCharge / step;
-        int k1 = (int)fmin(over, (V)(I - 1));
-        int k2 = (int)fmin((V)(k1 + 1), (V)(I - 1));
-        // the weights snap to {0, 1} (BoltzmannMC.C:959-967): row k1 has
-        // weight 1 unless k2 - over < 0.  A snapped pair picks one row, and
-        // 1 x + 0 x = x for the finite table values, so that row passed twice
-        // with weights (1, 0) gives the same numbers from one load per entry
-        const int kr = (V)k2 - over < (V)0 ? k2 : k1;
-        const V* cr = cumul + (size_t)kr * P;
-        const V* ir = interp + (size_t)kr * P;
-        V ref = (V)0;
-        if (L > 0) ref = lerp2((V)1, cr[L - 1], (V)0, cr[L - 1]);
-        V lim = prevSum + (lerp2((V)1, cr[R], (V)0, cr[R]) - ref) * rel;
-        if (randCS > lim) { prevSum = lim; continue; }
-        return channel_search(cr, cr, ir, ir, (V)1, (V)0, L, R, randCS, prevSum, ref, rel, true);
+    V prevSum = (V)0, rel = (V)0, sd = (V)0;
+    int row = -1, L = 0, R = 0;
+    constexpr int kBatch = 4;
+    for (int g0 = 0; g0 < G && row < 0; g0 += kBatch) {
+        V speed[kBatch], sum[kBatch];
+        int at[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const int g = g0 + k < G ? g0 + k : G - 1;
+            const ProcRec& pc = pr.proc[pr.gasFirst[g]];
+            const V dev = (V)pc.thermalStd;
+            V T[3];
+            for (int a = 0; a < 3; ++a) T[a] = vers[a] * dev;
+            V dx = e.vx - T[0], dy = e.vy - T[1], dz = e.vz - T[2];
+            speed[k] = sqrt(sqr_norm(dx, dy, dz));
+            V over = (V)0.5 * (V)pc.rMass * speed[k] * speed[k] / (V)kCharge / step;
+            int k1 = (int)fmin(over, (V)(I - 1));
+            int k2 = (int)fmin((V)(k1 + 1), (V)(I - 1));
+            // the weights snap to {0, 1} (BoltzmannMC.C:959-967): row k1 has
+            // weight 1 unless k2 - over < 0.  A snapped pair picks one row, and
+            // 1 x + 0 x = x for the finite table values, so that row passed twice
+            // with weights (1, 0) gives the same numbers from one load per entry
+            at[k] = (V)k2 - over < (V)0 ? k2 : k1;
+            sum[k] = gasSum[(size_t)at[k] * G + g];
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const int g = g0 + k;
+            if (g >= G || pr.gasFrac[g] == 0) continue;
+            const V lim = prevSum + sum[k] * speed[k];
+            if (row >= 0) continue;
+            if (randCS > lim) { prevSum = lim; continue; }
+            row = at[k];
+            rel = speed[k];
+            L = pr.gasFirst[g];
+            R = pr.gasLast[g];
+            sd = (V)pr.proc[L].thermalStd;
+        }
     }
-    return -1;
+    if (row < 0) return -1;
+    {
+#pragma clang fp contract(off)
+        for (int a = 0; a < 3; ++a) Vt[a] = vers[a] * sd;
+    }
+    const V* cr = cumul + (size_t)row * P;
+    const V* ir = interp + (size_t)row * P;
+    const V ref = L > 0 ? cr[L - 1] : (V)0;
+    return channel_search(cr, cr, ir, ir, (V)1, (V)0, L, R, randCS, prevSum, ref, rel, true);
 }
 
-// The collision operator of process `chosen` (BoltzmannMC.C:1101-1280).
+// The collision operator of process `chosen` (BoltzmannMC.C:1101-1280).  The
+// conservative collisions (cold, or with the target's thermal velocity) and
+// the ionizations of a wave share one sampler, azimuth and rotation.
 template <typename V, bool THERMAL>
 __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron<V>& e, EventRng<V>& rng,
                                                 CollOut<V>& o, int chosen, const V Vt[3], bool thermal) {
     o.pid = chosen;
+    rng.prime1();  // cos(chi) and the azimuth
     const ProcRec& pc = pr.proc[chosen];
     const int type = pc.type;
     const V inc = e.eps;
@@ -568,39 +615,17 @@ __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron
         o.dE = -(double)inc;  // attachmentCollision: the electron is lost
         return;
     }
-    if (THERMAL && thermal && type == 0) {
-        // conservativeCollision with the target's thermal velocity
-        double M = pc.tMass, mu = pc.rMass, loss = pc.energyLoss;
-        Sph<V> s;
-        if (!cart2sph(e.vx - Vt[0], e.vy - Vt[1], e.vz - Vt[2], s)) { o.flags |= ST_ZERO_VELOCITY; o.pid = -1; return; }
-        double relE = 0.5 * mu * (double)s.norm * (double)s.norm / kCharge;
-        double relAfter = relE - loss;
-        if (relAfter <= 0) { o.pid = -1; return; }
-        V cc = cos_chi<V>(pr, chosen, (V)relE, (V)relAfter, rng, 6);
-        V sc = sin_chi(cc);
-        V se, ce;
-        turn_sincos(rng.u(7), se, ce);
-        V u[3];
-        euler(sc, cc, se, ce, s, u);
-        double rel2 = (double)s.norm * (double)s.norm - 2.0 / mu * loss * kCharge;
-        if (!(rel2 > 0)) { o.pid = -1; return; }  // rounding at the threshold edge
-        V sp = (V)sqrt(rel2);
-        V fM = (V)(M / (kMass + M)), fe = (V)(kMass / (kMass + M));
-        e.vx = fM * (sp * u[0]) + (fe * e.vx + fM * Vt[0]);
-        e.vy = fM * (sp * u[1]) + (fe * e.vy + fM * Vt[1]);
-        e.vz = fM * (sp * u[2]) + (fe * e.vz + fM * Vt[2]);
-        e.eps = energy_of(e.vx, e.vy, e.vz);
-        o.dE = (double)e.eps - (double)inc;
-        return;
-    }
-    // conservativeCollision (cold) and ionizationCollision share the
-    // scattering of the incident electron: one sampler, azimuth and rotation
     const bool ion = type == 1;
+    const bool moving = THERMAL && thermal && !ion;  // the target moves: scattering of the relative velocity
     const double loss = pc.energyLoss;  // energy loss, or the ionization threshold
     if (ion && (double)inc < loss) { o.pid = -1; return; }
     Sph<V> s;
-    if (!cart2sph(e.vx, e.vy, e.vz, s)) { o.flags |= ST_ZERO_VELOCITY; o.pid = -1; return; }
-    const double after = (double)inc - loss;  // energy after the loss; net energy of an ionization
+    const bool moves = moving ? cart2sph(e.vx - Vt[0], e.vy - Vt[1], e.vz - Vt[2], s) : cart2sph(e.vx, e.vy, e.vz, s);
+    if (!moves) { o.flags |= ST_ZERO_VELOCITY; o.pid = -1; return; }
+    const double M = pc.tMass, mu = pc.rMass;
+    double before = (double)inc;
+    if (moving) before = 0.5 * mu * (double)s.norm * (double)s.norm / kCharge;
+    const double after = before - loss;  // energy after the loss; net energy of an ionization
     if (!ion && after <= 0) { o.pid = -1; return; }
     const V net = (V)after;
     V ej = (V)0, scE = net;
@@ -618,7 +643,7 @@ __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron
     const bool boeuf = ion && pc.scat == 5;
     V cc;
     if (boeuf) cc = sqrt(scE / net);
-    else cc = cos_chi<V>(pr, chosen, inc, scE, rng, 6);
+    else cc = cos_chi<V>(pr, chosen, (V)before, scE, rng, 6);
     const V sc = sin_chi(cc);
     V se, ce;
     turn_sincos(rng.u(7), se, ce);
@@ -627,13 +652,23 @@ __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron
     V sp;
     if (ion) {
         sp = sqrt((V)2 * scE * (V)kCharge / (V)kMass);
+    } else if (moving) {
+        double rel2 = (double)s.norm * (double)s.norm - 2.0 / mu * loss * kCharge;
+        if (!(rel2 > 0)) { o.pid = -1; return; }  // rounding at the threshold edge
+        sp = (V)sqrt(rel2);
     } else {
-        const double M = pc.tMass, mu = pc.rMass;
         double v2after = (double)s.norm * (double)s.norm - 2.0 / kMass * loss * kCharge;
         if (!(v2after > 0)) { o.pid = -1; return; }  // rounding at the threshold edge
         sp = sqrt((V)v2after * ((V)1 - (V)(2.0 * mu / (kMass + M)) * ((V)1 - cc)));
     }
-    e.vx = sp * u[0]; e.vy = sp * u[1]; e.vz = sp * u[2];
+    if (moving) {
+        V fM = (V)(M / (kMass + M)), fe = (V)(kMass / (kMass + M));
+        e.vx = fM * (sp * u[0]) + (fe * e.vx + fM * Vt[0]);
+        e.vy = fM * (sp * u[1]) + (fe * e.vy + fM * Vt[1]);
+        e.vz = fM * (sp * u[2]) + (fe * e.vz + fM * Vt[2]);
+    } else {
+        e.vx = sp * u[0]; e.vy = sp * u[1]; e.vz = sp * u[2];
+    }
     if (!ion) {
         e.eps = energy_of(e.vx, e.vy, e.vz);
         o.dE = (double)e.eps - (double)inc;
@@ -667,11 +702,12 @@ template <typename V, bool THERMAL>
 __device__ inline void collide(const CondParams& c, const DevProcesses& pr, const V* cumul, const V* interp,
                                const V* nutot, Electron<V>& e, EventRng<V>& rng, CollOut<V>& o) {
     clear_out(o);
+    const V* gasSum = nutot + c.I + 2 * kEnvBins;
     V Vt[3] = {(V)0, (V)0, (V)0};
     const bool thermal = THERMAL && is_thermal(c, pr, e);
     int chosen;
     if (THERMAL && thermal) {
-        chosen = thermal_choose(c, pr, cumul, interp, e, rng, Vt);
+        chosen = thermal_choose(c, pr, cumul, interp, gasSum, e, rng, Vt);
         if (chosen == -1) return;
     } else {
         if (!cold_null_test(c, nutot, e, rng, o)) return;
@@ -694,10 +730,12 @@ __device__ __forceinline__ int step_a(const CondParams& c, const DevProcesses& p
                                       const V* envLo, Electron<V>& e, EventRng<V>& rng, CollOut<V>& o,
                                       double& gain) {
     if (e.t == c.tsync) return STEP_DONE;
-    const bool pending = e.tfree < (V)0;  // pending free time undefined (NON_DEF is negative)
-    if (pending || e.t + (double)e.tfree <= c.tsync) rng.prime0();
-    if (pending) {
-        e.tfree = free_time(rng.u(0), c);
+    // the draws of every lane, whether it needs a free time, a variate of the
+    // null test or neither (a pending flight that outlasts the interval)
+    rng.prime0();
+    const V fresh = free_time(rng.u(0), c);
+    if (e.tfree < (V)0) {  // pending free time undefined (NON_DEF is negative)
+        e.tfree = fresh;
         e.nue = (V)c.trial;
     }
     // one flight for both outcomes (a wave holds both kinds of lanes)
@@ -724,13 +762,13 @@ __device__ __forceinline__ int step_a(const CondParams& c, const DevProcesses& p
 
 template <typename V, bool THERMAL>
 __device__ __forceinline__ void step_b(const CondParams& c, const DevProcesses& pr, const V* cumul, const V* interp,
-                                       Electron<V>& e, EventRng<V>& rng, CollOut<V>& o) {
+                                       const V* gasSum, Electron<V>& e, EventRng<V>& rng, CollOut<V>& o) {
     clear_out(o);
     V Vt[3] = {(V)0, (V)0, (V)0};
     const bool thermal = THERMAL && is_thermal(c, pr, e);
     int chosen;
     if (THERMAL && thermal) {
-        chosen = thermal_choose(c, pr, cumul, interp, e, rng, Vt);
+        chosen = thermal_choose(c, pr, cumul, interp, gasSum, e, rng, Vt);
         if (chosen == -1) return;
     } else {
         chosen = cold_choose(c, pr, cumul, interp, e, rng);

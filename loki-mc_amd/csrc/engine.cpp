@@ -471,7 +471,7 @@ public:
             cp.N = cs[c].N;
             cp.gasEnergy = cs[c].gasEnergy;
             cp.seed = num.seed ^ ((uint64_t)c * 0x9E3779B97F4A7C15ull);
-            cp.tableOffset = (int64_t)c * table_block_size(I, P);
+            cp.tableOffset = (int64_t)c * table_block_size(I, P, pl.G);
             cp.envShift = envShift;
             cp.base = base;
             cp.nMain = Nc;
@@ -505,7 +505,7 @@ public:
         HIP_TRY(alive.alloc(capacity));
         HIP_TRY(holeList.alloc(capacity));
         HIP_TRY(hipMemsetAsync(alive.p, 0, capacity, stream));
-        HIP_TRY(tables.alloc((size_t)n * table_block_size(I, P)));
+        HIP_TRY(tables.alloc((size_t)n * table_block_size(I, P, pl.G)));
         HIP_TRY(dconds.alloc(n));
         HIP_TRY(chunks.alloc(nChunks));
         HIP_TRY(hipMemcpyAsync(chunks.p, hchunks.data(), nChunks * sizeof(Chunk), hipMemcpyHostToDevice, stream));
@@ -629,7 +629,8 @@ public:
             HIP_TRY(tsrcI.alloc(ti.size()));
             HIP_TRY(hipMemcpy(tsrcD.p, td.data(), td.size() * sizeof(double), hipMemcpyHostToDevice));
             HIP_TRY(hipMemcpy(tsrcI.p, ti.data(), ti.size() * sizeof(int), hipMemcpyHostToDevice));
-            tsrc.P = P; tsrc.I = I;
+            tsrc.P = P; tsrc.I = I; tsrc.G = pl.G;
+            tsrc.gasFirst = iproc.p; tsrc.gasLast = iproc.p + pl.G;
             tsrc.energy = tsrcD.p; tsrc.sigma = tsrcD.p + nPts;
             const double* pd = tsrcD.p + 2 * nPts;
             tsrc.minE = pd; tsrc.maxE = pd + P; tsrc.relDens = pd + 2 * P; tsrc.statW = pd + 3 * P;

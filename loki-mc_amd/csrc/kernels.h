@@ -196,7 +196,9 @@ struct FlightLists {
 // (a superelastic process reads its inelastic partner's) and the constants of
 // the interpolation.
 struct DevTableSrc {
-    int P, I;
+    int P, I, G;
+    const int* gasFirst;       // [G] process range of each gas
+    const int* gasLast;
     const double* energy;      // concatenated prepared tables
     const double* sigma;
     const int* srcBegin;       // [P] first point of the table process p reads
@@ -212,13 +214,14 @@ struct DevTableSrc {
 // Build condition tables on the device for gas density N and energy step
 // `step` (= max energy / (I-1)): `tables` receives cumul [I*P], interp [I*P],
 // nutot [I], then the null-test envelope envHi [kEnvBins], envLo [kEnvBins]
-// over bins of 1 << envShift rows, in V; nutot64 [I] and numax64 [I]
+// over bins of 1 << envShift rows, and the sum over each gas's processes
+// gasSum [I*G], in V; nutot64 [I] and numax64 [I]
 // (running maximum) in FP64.
 template <typename V>
 hipError_t launch_tables(const DevTableSrc& src, double N, double step, int envShift, V* tables,
                          double* nutot64, double* numax64, hipStream_t st);
 // Elements of one condition's table block.
-inline int64_t table_block_size(int I, int P) { return (int64_t)I * (2 * P + 1) + 2 * kEnvBins; }
+inline int64_t table_block_size(int I, int P, int G) { return (int64_t)I * (2 * P + 1 + G) + 2 * kEnvBins; }
 
 // mainBase[c]: index of condition c's first electron among all main electrons
 template <typename V>

@@ -658,7 +658,7 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
         if (pk && (__popcll(pk) >= pr.parkLanes || pk == (live & ~__ballot(done)))) {
             if (parked) {
                 EventRng<V> rng(cp.seed, e.stream, e.event, c0);
-                step_b<V, THERMAL>(cp, pr, cumul, interp, e, rng, o);
+                step_b<V, THERMAL>(cp, pr, cumul, interp, nutot + I + 2 * kEnvBins, e, rng, o);
                 status |= o.flags;
                 if (o.pid < 0) {
                     ++nNull;
@@ -1645,6 +1645,7 @@ __global__ __launch_bounds__(kBlock) void k_table_rows(DevTableSrc a, double N, 
     V* cumul = tables;
     V* interp = tables + (size_t)I * P;
     V* nutot = interp + (size_t)I * P;
+    V* gasSum = nutot + I + 2 * kEnvBins;
     for (int q = threadIdx.x; q < rows * P; q += kBlock) {
         const int i = i0 + q / P;
         if (i >= I) break;
@@ -1660,6 +1661,11 @@ __global__ __launch_bounds__(kBlock) void k_table_rows(DevTableSrc a, double N, 
         for (int p = 0; p < P; ++p) {
             acc += vals[r * P + p];
             cumul[(size_t)i * P + p] = (V)acc;
+        }
+        for (int g = 0; g < a.G; ++g) {
+            const int L = a.gasFirst[g];
+            const V below = L > 0 ? cumul[(size_t)i * P + L - 1] : (V)0;
+            gasSum[(size_t)i * a.G + g] = cumul[(size_t)i * P + a.gasLast[g]] - below;
         }
         acc *= N * sqrt(i * step * 2.0 * kCharge / kMass);
         nutot[i] = (V)acc;

@@ -491,23 +491,26 @@ __device__ __forceinline__ bool cold_null_test(const CondParams& c, const V* nut
 
 // The same decision with the per-bin envelope envHi/envLo of the total
 // frequency (bounds of every interpolated value a bin's rows can give,
-// widened by a few ulp): only a variate between the bounds reads the table.
-// The result, and the escape flag, equal those of cold_null_test.
+// widened by a few ulp): only a variate between the bounds reads the table, and
+// only for a lane with `want`.  The result, and the escape flag, equal those of
+// cold_null_test.
 template <typename V>
 __device__ __forceinline__ bool cold_null_test_env(const CondParams& c, const V* nutot, const V* envHi,
                                                    const V* envLo, const Electron<V>& e, EventRng<V>& rng,
-                                                   CollOut<V>& o) {
+                                                   bool want, bool& escape) {
     const ColdRow<V> r = cold_row(c, e);
     const V randF = e.nue * rng.u(5);
     const int bin = r.k1 >> c.envShift;
     const V hi = envHi[bin], lo = envLo[bin];
-    const bool needTot = (randF > lo && !(randF > hi)) || e.nue < hi;
-    V tot = hi;
-    if (needTot) tot = lerp2(r.w1, nutot[r.k1], r.w2, nutot[r.k2]);
-    o.escape = needTot ? e.nue < tot : false;
-    if (randF > hi) return false;
-    if (!(randF > lo)) return true;
-    return !(randF > tot);
+    const bool over = randF > hi, clear = randF > lo;
+    escape = false;
+    bool real = !clear;
+    if (want && ((clear && !over) || e.nue < hi)) {
+        const V tot = lerp2(r.w1, nutot[r.k1], r.w2, nutot[r.k2]);
+        escape = e.nue < tot;
+        real = !over && (!clear || !(randF > tot));
+    }
+    return real;
 }
 
 // Cold channel choice of a real collision (BoltzmannMC.C:1055-1097)
@@ -723,23 +726,31 @@ __device__ inline void collide(const CondParams& c, const DevProcesses& pr, cons
 // call 0 of the electron's current event), fly to t_sync or to the collision
 // and, in the cold branch, run the null test.  Phase B: the channel choice
 // and collision operator of a real (or thermal) collision.
+// An electron at t_sync (a collision or an ejection exactly there) flies for no
+// time, which changes nothing, and keeps its pending or undefined free time.
+// Every lane runs the same instructions to the end: what differs between a
+// flight that ends at t_sync and one that ends in a null or a real collision is
+// selected, not branched on.  (The step's flights are the largest part of a
+// wave's time, 44 % on the 64-condition scan, and a third of their instructions
+// kept lane masks: flight kernel per interval, branching against this, 861 ->
+// 830 us for that scan in mixed precision and 1373 -> 1359 in FP64, one condition
+// of 1e4 electrons 47.7 -> 44.5, of 1e8 with thermal targets 14.6 -> 14.1 ms.)
 enum StepResult { STEP_DONE = 1, STEP_NULL = 2, STEP_REAL = 3 };
 
 template <typename V, int FC, bool THERMAL>
 __device__ __forceinline__ int step_a(const CondParams& c, const DevProcesses& pr, const V* nutot, const V* envHi,
-                                      const V* envLo, Electron<V>& e, EventRng<V>& rng, CollOut<V>& o,
+                                      const V* envLo, Electron<V>& e, EventRng<V>& rng, bool& escape,
                                       double& gain) {
-    if (e.t == c.tsync) return STEP_DONE;
     // the draws of every lane, whether it needs a free time, a variate of the
     // null test or neither (a pending flight that outlasts the interval)
     rng.prime0();
     const V fresh = free_time(rng.u(0), c);
-    if (e.tfree < (V)0) {  // pending free time undefined (NON_DEF is negative)
-        e.tfree = fresh;
-        e.nue = (V)c.trial;
-    }
+    const bool idle = e.t == c.tsync;
+    const bool draw = e.tfree < (V)0 && !idle;  // pending free time undefined (NON_DEF is negative)
+    e.tfree = draw ? fresh : e.tfree;
+    e.nue = draw ? (V)c.trial : e.nue;
     // one flight for both outcomes (a wave holds both kinds of lanes)
-    const bool partial = e.t + (double)e.tfree > c.tsync;
+    const bool partial = idle || e.t + (double)e.tfree > c.tsync;
     const double dt = partial ? c.tsync - e.t : (double)e.tfree;
     if (FC == FLIGHT_DC_ANY) {
         if (c.fieldCase == FIELD_DC) flight<FIELD_DC>(c, e, dt, gain);
@@ -747,17 +758,12 @@ __device__ __forceinline__ int step_a(const CondParams& c, const DevProcesses& p
     } else {
         flight<FC>(c, e, dt, gain);
     }
-    if (partial) {
-        e.t = c.tsync;
-        e.tfree = (V)((double)e.tfree - dt);
-        return STEP_DONE;
-    }
-    e.t += (double)e.tfree;
-    if (THERMAL && is_thermal(c, pr, e)) {
-        o.escape = false;  // only the cold null test compares the trial frequency with the total
-        return STEP_REAL;
-    }
-    return cold_null_test_env(c, nutot, envHi, envLo, e, rng, o) ? STEP_REAL : STEP_NULL;
+    e.t = partial ? c.tsync : e.t + dt;
+    e.tfree = partial ? (V)((double)e.tfree - dt) : e.tfree;
+    const bool thermal = THERMAL && is_thermal(c, pr, e);
+    // only the cold null test compares the trial frequency with the total
+    const bool real = cold_null_test_env(c, nutot, envHi, envLo, e, rng, !partial && !thermal, escape);
+    return partial ? STEP_DONE : (thermal || real ? STEP_REAL : STEP_NULL);
 }
 
 template <typename V, bool THERMAL>

@@ -622,34 +622,30 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
         // event is a null collision flies on in the same step, up to null_run<V>()
         // events (the draws are keyed by the event, so the run length changes
         // no trajectory)
-        if (have && !parked) {
-            for (int run = 0; run < null_run<V>(); ++run) {
-                double gain = 0;
-                EventRng<V> rng(cp.seed, e.stream, e.event);
-                const int st = step_a<V, FC, THERMAL>(cp, pr, nutot, envHi, envLo, e, rng, o, gain);
-                fieldGain += gain;
-                if (st == STEP_DONE) {
-                    done = true;
-                    break;
-                }
-                if (!isfinite(e.t) || !isfinite((double)e.eps)) {
-                    status |= ST_NONFINITE;
-                    e.t = cp.tsync;
-                    done = true;
-                    break;
-                }
-                if (o.escape) ++nEsc;
-                if (st != STEP_NULL) {
-                    parked = true;
-                    c0[0] = rng.w0[0]; c0[1] = rng.w0[1]; c0[2] = rng.w0[2]; c0[3] = rng.w0[3];
-                    break;
-                }
+        bool fly = have && !parked;
+#pragma unroll
+        for (int run = 0; run < null_run<V>(); ++run) {
+            if (!fly) continue;
+            double gain = 0;
+            bool escape;
+            EventRng<V> rng(cp.seed, e.stream, e.event);
+            const int st = step_a<V, FC, THERMAL>(cp, pr, nutot, envHi, envLo, e, rng, escape, gain);
+            fieldGain += gain;
+            const bool bad = st != STEP_DONE && (!isfinite(e.t) || !isfinite((double)e.eps));
+            status |= bad ? (uint32_t)ST_NONFINITE : 0u;
+            e.t = bad ? cp.tsync : e.t;
+            nEsc += escape && !bad ? 1u : 0u;
+            c0[0] = rng.w0[0]; c0[1] = rng.w0[1]; c0[2] = rng.w0[2]; c0[3] = rng.w0[3];
+            done = st == STEP_DONE || bad;
+            parked = st == STEP_REAL && !bad;
+            fly = st == STEP_NULL && !bad;
+            if (fly) {
                 ++nNull;
                 after_event(cp, e);
                 if (++iter >= kMaxLoopPerSync) {
                     status |= ST_LOOP_CAP;
                     done = true;
-                    break;
+                    fly = false;
                 }
             }
         }

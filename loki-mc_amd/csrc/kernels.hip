@@ -136,6 +136,61 @@ template <typename V> __device__ __forceinline__ void store_rec(const DevState<V
     draw_part(q).nue = e.nue; draw_part(q).event = e.event; draw_part(q).stream = e.stream;
     rec_put(s, i, q);
 }
+// A value of the lane that quad_perm CTRL names, within each four lanes.
+template <int CTRL> __device__ __forceinline__ uint32_t quad_get(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+}
+// Lanes 2k and 2k + 1 (XOR 1), or k and k + 2 of four (XOR 2), exchange: the lower
+// keeps a and gets the upper's a in b, the upper keeps b and gets the lower's b in a.
+template <int XOR> __device__ __forceinline__ void lane_swap(uint4& a, uint4& b, bool upper) {
+    constexpr int ctrl = XOR == 1 ? 0xB1 : 0x4E;  // quad_perm 1,0,3,2 / 2,3,0,1
+    uint32_t x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t xo = quad_get<ctrl>(x[k]), yo = quad_get<ctrl>(y[k]);
+        x[k] = upper ? yo : x[k];
+        y[k] = upper ? y[k] : xo;
+    }
+    a = make_uint4(x[0], x[1], x[2], x[3]);
+    b = make_uint4(y[0], y[1], y[2], y[3]);
+}
+template <int J> __device__ __forceinline__ void store_quad(char* base, uint32_t slot, const uint4& v, int lane) {
+    const uint32_t to = quad_get<J * 0x55>(slot);
+    if (to != 0xffffffffu) *(uint4*)(base + ((size_t)to * 64 + (lane & 3) * 16)) = v;
+}
+// Store the records of the lanes with `put` (called by a whole wave).  A lane
+// storing its own record writes 16 bytes to each of 64 places per instruction,
+// four L2 writes per record; here the lanes of four exchange pieces first, so
+// that each instruction writes whole 64-byte records, four lanes to a record.
+// The exchange is about 50 instructions a step; it pays where the chip is full
+// of waves and the L2 writes are what they wait for, so for the mixed form in
+// launches with more chunks than waves.  Flight kernel per interval, own record
+// against this: 64-condition scan 827 -> 784 us, one condition of 3e7 electrons
+// 1324 -> 1234, 24 AC conditions of 2e5 635 -> 620; but one condition of 1e4
+// 43.9 -> 46.6, eight of 1e5 (a wave per chunk) 137 -> 145, one of 1e8 with
+// thermal targets (bound by the collision step) 14.1 -> 14.3 ms, and the FP64
+// form, whose record has a second part of 32 bytes, 2341 -> 2450 for one of 3e7.
+template <typename V>
+__device__ __forceinline__ void store_recs(const DevState<V>& s, bool put, int64_t slot, const Electron<V>& e) {
+    Rec<V> q = {};
+    q.a.x = e.x; q.a.y = e.y; q.a.z = e.z; q.a.t = e.t;
+    q.a.vx = e.vx; q.a.vy = e.vy; q.a.vz = e.vz; q.a.tfree = e.tfree;
+    draw_part(q).nue = e.nue; draw_part(q).event = e.event; draw_part(q).stream = e.stream;
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t to = put ? (uint32_t)slot : 0xffffffffu;  // the pool has less than 2^32 - 16 slots
+    static_assert(sizeof(q.a) == 64, "four pieces");
+    uint4 p[4];
+    __builtin_memcpy(p, &q.a, 64);
+    lane_swap<1>(p[0], p[1], lane & 1);
+    lane_swap<1>(p[2], p[3], lane & 1);
+    lane_swap<2>(p[0], p[2], lane & 2);
+    lane_swap<2>(p[1], p[3], lane & 2);
+    char* base = (char*)s.ra;
+    store_quad<0>(base, to, p[0], lane);
+    store_quad<1>(base, to, p[1], lane);
+    store_quad<2>(base, to, p[2], lane);
+    store_quad<3>(base, to, p[3], lane);
+}
 template <typename V> __device__ __forceinline__ double rec_energy(const RecA<V>& q) {
     return (double)energy_of(q.vx, q.vy, q.vz);
 }
@@ -510,7 +565,7 @@ __device__ __forceinline__ void hist_count(const DevHist& h, int c, const double
 template <typename V, int FC, bool THERMAL, int HIST>
 __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWork& w, const DevProcesses& pr,
                                               const V* tables, const DevHist& h, int cid, unsigned long long* cnt,
-                                              lds_uint4* ring) {
+                                              lds_uint4* ring, bool lines) {
     const int lane = lane_id();
     const int P = pr.P;
     long long* gainL = (long long*)(cnt + P);
@@ -548,6 +603,7 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
     int nextMain = 0, nq = 0, nextNew = 0, holes = 0;
     int loaded = 0;  // main records whose ring loads are issued
     int landed = 0;  // ring fills known to have landed
+    constexpr bool kLines = !split_record<V>() && !THERMAL;
     constexpr int kAhead = (ring_segs<V>() - 1) * kRingSeg;
     for (; loaded < count && loaded <= nextMain + kAhead; loaded += kRingSeg)
         ring_fill<V, kPairFill>(s, ch.first, count, loaded, ring);
@@ -696,12 +752,13 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
         }
         // finished electrons: store, or leave a hole in the chunk's list
         const uint64_t dm = __ballot(done && dead && !isNew);
+        if (kLines && lines) store_recs(s, done && !dead, slot, e);
         if (done) {
             if (dead) {
                 s.alive[slot] = 0;
                 if (!isNew) w.holeList[ch.first + holes + lane_rank(dm)] = (uint32_t)slot;
             } else {
-                store_rec(s, slot, e);
+                if (!(kLines && lines)) store_rec(s, slot, e);
                 maxE = fmax(maxE, (double)e.eps);
             }
             have = false;
@@ -805,7 +862,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_w
             if (fl.oneShot || x == xcd) break;
             continue;
         }
-        advance_chunk<V, FC, THERMAL, HIST>(s, w, prl, tables, h, fl.list[item], cnt, ring);
+        advance_chunk<V, FC, THERMAL, HIST>(s, w, prl, tables, h, fl.list[item], cnt, ring, !fl.oneShot);
         if (fl.oneShot) break;
     }
 }

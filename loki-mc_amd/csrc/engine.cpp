@@ -234,6 +234,22 @@ double max_accel_energy(const Cond& c, double initialEnergy, double deltaT) {
     return initialEnergy + g;
 }
 
+// A batch of at least kPartElectrons electrons runs in two parts, and the
+// flight launch of a part that queues its chunks takes kPartShare / 8 of the
+// waves that fit, so that the other part's kernels find room beside it.  Passes,
+// one part against two (16 or 32 intervals): the 64-condition scan of 1.6e7
+// electrons, mixed 17.8 -> 16.9 ms, FP64 27.0 -> 24.2; 32 conditions of N2-like gas
+// (1e7) mixed 11.5 -> 10.7, FP64 17.1 -> 15.3; 24 AC conditions of 2e5 12.3 -> 10.9;
+// eight of 1e5 7.1 -> 6.7; six of 5e5 in all mixed 5.3 -> 5.1, FP64 6.1 -> 5.4.  Below
+// that the host's turns are what takes the time: eight of 2.6e5 in all 4.51 ->
+// 4.46, four ECR conditions of 2.4e5 in all 5.21 -> 5.36.  With all of the waves
+// the FP64 scan took 26.2 ms, with 3/4 of them 24.8 (mixed 16.7, 17.1); three parts
+// took the mixed scan to 16.3, but four streams of one process share the
+// hardware's queues and are slower than one part (19.3).
+constexpr int kMaxParts = 2;
+constexpr int64_t kPartElectrons = 400000;
+constexpr int kPartShare = 7;
+
 // =============================================================== Engine<V>
 template <typename V> class Engine : public EngineBase {
 public:
@@ -258,12 +274,10 @@ public:
     DevBuf<int32_t> gCond, gFirst, gCount, cGroup, cGroups;  // reduction groups (huge conditions)
     DevBuf<double> tailG, momG;
     int nGroups = 0;
+    std::vector<int32_t> hGroup;  // first reduction group of each condition
     DevBuf<unsigned long long> accCount;
     DevBuf<long long> accGain, accLoss;
     DevBuf<PopPlan> plans;
-    FlightLists fl = {};
-    std::vector<int32_t> listActive;  // active flags the flight lists were built for
-    int listAge = 0;                  // intervals since the flight lists were ordered
     // histogram grid and phase rows as last uploaded (staged in pinned memory)
     PinnedBuf<double> pinGrid;
     PinnedBuf<int32_t> pinRow;
@@ -290,21 +304,50 @@ public:
     DevBuf<int> tsrcI;
     DevTableSrc tsrc = {};
     DevBuf<SlotRange> ranges;
-    KernelTimer timer;
-    // the cycle after the flights as a HIP graph (captured at the first
-    // interval, replayed at every later one)
+    // A part of the batch whose intervals run on a stream of its own: a range of
+    // conditions.  Conditions do not depend on each other, so while one part's
+    // interval is summed up on the host, the other part's kernels run, and a
+    // part's population control and sampling fill the chip while the last
+    // waves of the other part's flights leave it.
+    struct Part {
+        int c0 = 0, c1 = 0;               // conditions
+        hipStream_t stream = nullptr;
+        DevWork dw = {};
+        DevHist dh = {};                  // its histogram ranges
+        FlightLists fl = {};
+        std::vector<int32_t> hlist;
+        std::vector<int32_t> listActive;  // active flags the flight lists were built for
+        bool listMerged = false;          // with DC and DC+B conditions in one launch
+        int listAge = 0;                  // intervals since the flight lists were ordered
+        KernelTimer timer = {};
+        hipEvent_t flightBefore[2] = {};  // the flight events of the interval before (start, stop)
+        bool countsInterval = false;      // the first part of the interval in flight
+        bool inFlight = false;            // an interval is launched and not yet summed up
+        // the cycle after the flights as a HIP graph (captured at the first
+        // interval, replayed at every later one)
+        hipGraph_t cycGraph = nullptr;
+        hipGraphExec_t cycExec = nullptr;
+    };
+    std::vector<Part> parts;
+    hipStream_t cur = nullptr;          // stream of the part being prepared or summed up
+    hipEvent_t lastFlight = nullptr;    // end of the flights last counted
+    int timerLevel = 1;
     bool useGraph = true;
-    hipGraph_t cycGraph = nullptr;
-    hipGraphExec_t cycExec = nullptr;
 
     ~Engine() override {
         if (stream) (void)hipStreamSynchronize(stream);
         set_kernel_timer(nullptr);
-        if (cycExec) (void)hipGraphExecDestroy(cycExec);
-        if (cycGraph) (void)hipGraphDestroy(cycGraph);
-        for (int k = 0; k < K_COUNT; ++k) {
-            if (timer.start[k]) (void)hipEventDestroy(timer.start[k]);
-            if (timer.stop[k]) (void)hipEventDestroy(timer.stop[k]);
+        for (Part& p : parts) {
+            if (p.stream) (void)hipStreamSynchronize(p.stream);
+            if (p.cycExec) (void)hipGraphExecDestroy(p.cycExec);
+            if (p.cycGraph) (void)hipGraphDestroy(p.cycGraph);
+            for (int k = 0; k < K_COUNT; ++k) {
+                if (p.timer.start[k]) (void)hipEventDestroy(p.timer.start[k]);
+                if (p.timer.stop[k]) (void)hipEventDestroy(p.timer.stop[k]);
+            }
+            for (hipEvent_t e : p.flightBefore)
+                if (e) (void)hipEventDestroy(e);
+            if (p.stream && p.stream != stream) (void)hipStreamDestroy(p.stream);
         }
         recA.release(); recB.release(); holeList.release(); pop.release(); laneMarks.release(); status.release(); queue.release();
         alive.release(); tables.release(); dconds.release(); chunks.release(); holesC.release();
@@ -350,11 +393,7 @@ public:
         if (hipGetDeviceCount(&dev) != hipSuccess || dev == 0) return fail(EKMC_ERR_NO_DEVICE, "no HIP device is visible");
         HIP_TRY(hipGetDevice(&device));
         HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-        for (int k = 0; k < K_COUNT; ++k) {
-            HIP_TRY(hipEventCreate(&timer.start[k]));
-            HIP_TRY(hipEventCreate(&timer.stop[k]));
-            timer.armed[k] = false;
-        }
+        cur = stream;
         // EKMC_FUSED_HIST=0: every histogram by the histogram kernel
         const char* fh = std::getenv("EKMC_FUSED_HIST");
         fusedHist = !(fh && fh[0] == '0');
@@ -370,7 +409,7 @@ public:
         // HIP-event timing of the flight kernels; EKMC_KERNEL_TIMING=all times
         // every kernel, EKMC_KERNEL_TIMING=0 none
         const char* kt = std::getenv("EKMC_KERNEL_TIMING");
-        timer.level = !kt ? 1 : (std::strcmp(kt, "all") == 0 ? 2 : (kt[0] == '0' ? 0 : 1));
+        timerLevel = !kt ? 1 : (std::strcmp(kt, "all") == 0 ? 2 : (kt[0] == '0' ? 0 : 1));
         kstat.assign(K_COUNT + H_COUNT, {0, 0.0});
         cs.assign(n, Cond());
         int64_t sumN = 0;
@@ -542,6 +581,7 @@ public:
                     cn[c] = (int32_t)gc.size() - cg[c];
                 }
                 nGroups = (int)gc.size();
+                hGroup = cg;
                 HIP_TRY(gCond.alloc(nGroups)); HIP_TRY(gFirst.alloc(nGroups)); HIP_TRY(gCount.alloc(nGroups));
                 HIP_TRY(cGroup.alloc(n)); HIP_TRY(cGroups.alloc(n));
                 HIP_TRY(tailG.alloc((size_t)nGroups * CT_SIZE)); HIP_TRY(momG.alloc((size_t)nGroups * kMomentRecord));
@@ -558,7 +598,7 @@ public:
         HIP_TRY(hipMemsetAsync(accCount.p, 0, (size_t)n * P * 8, stream));
         HIP_TRY(hipMemsetAsync(accGain.p, 0, (size_t)n * P * 8, stream));
         HIP_TRY(hipMemsetAsync(accLoss.p, 0, (size_t)n * P * 8, stream));
-        HIP_TRY(queue.alloc(kFlightClasses * kXcds * kQueueStride));
+        HIP_TRY(queue.alloc(kMaxParts * kFlightClasses * kXcds * kQueueStride));
         HIP_TRY(hipMemsetAsync(queue.p, 0, queue.n * sizeof(uint32_t), stream));
         HIP_TRY(plans.alloc(n));
         HIP_TRY(status.alloc(n));
@@ -661,15 +701,10 @@ public:
         dw.holeList = holeList.p; dw.laneMarks = laneMarks.p; dw.pop = pop.p; dw.tailC = tailC.p; dw.momC = momC.p; dw.accCount = accCount.p;
         dw.accGain = accGain.p; dw.accLoss = accLoss.p; dw.plans = plans.p;
         dw.status = status.p; dw.queue = queue.p; dw.summary = summary.p; dw.summarySize = summarySize;
-        dw.recSize = recSize; dw.nChunks = nChunks; dw.nCond = n;
+        dw.recSize = recSize; dw.chunk0 = 0; dw.nChunks = nChunks; dw.cond0 = 0; dw.nCond = n; dw.group0 = 0;
         dw.groupCond = gCond.p; dw.groupFirst = gFirst.p; dw.groupCount = gCount.p;
         dw.condGroup = cGroup.p; dw.condGroups = cGroups.p; dw.tailG = tailG.p; dw.momG = momG.p;
         dw.nGroups = nGroups;
-        dw.planMarks = dw.planPairs = 0;
-        for (int c = 0; c < n; ++c) {
-            if (hcp[c].nMain > kPlanDirect) dw.planMarks = 1;
-            if (hcp[c].nChunks > kPairsDirect) dw.planPairs = 1;
-        }
         dh.eedf = hEedf.p; dh.eedfPer = hPer.p; dh.eadf = hEadf.p; dh.evdf = hEvdf.p; dh.grid = grid.p;
         dh.evdf3 = hEvdf3.p; dh.n3 = n3;
         dh.phaseRow = phaseRow.p; dh.cyl = cylFlag.p;
@@ -723,7 +758,63 @@ public:
         HIP_TRY(hipMemcpy(ranges.p, hr.data(), hr.size() * sizeof(SlotRange), hipMemcpyHostToDevice));
         dh.ranges = ranges.p;
         dh.nRanges = (int)hr.size();
+        ekmc_status ps = create_parts(hr);
+        if (ps != EKMC_OK) return ps;
         HIP_TRY(hipStreamSynchronize(stream));
+        return EKMC_OK;
+    }
+
+    // The parts of the batch: two of about as many electrons where the batch
+    // has kPartElectrons, else one.
+    ekmc_status create_parts(const std::vector<SlotRange>& hr) {
+        std::vector<int> cut = {0, nCond};
+        if (nCond > 1 && totalMain >= kPartElectrons && timerLevel < 2) {
+            int64_t sum = 0;
+            int c = 0;
+            while (c + 1 < nCond && 2 * (sum + hcp[c].nMain / 2) < totalMain) sum += hcp[c++].nMain;
+            cut.insert(cut.begin() + 1, std::max(c, 1));
+        }
+        parts.resize(cut.size() - 1);
+        for (size_t i = 0; i < parts.size(); ++i) {
+            Part& p = parts[i];
+            p.c0 = cut[i];
+            p.c1 = cut[i + 1];
+            p.stream = stream;
+            if (i > 0) {
+                p.stream = nullptr;
+                HIP_TRY(hipStreamCreateWithFlags(&p.stream, hipStreamNonBlocking));
+            }
+            for (int k = 0; k < K_COUNT; ++k) {
+                HIP_TRY(hipEventCreate(&p.timer.start[k]));
+                HIP_TRY(hipEventCreate(&p.timer.stop[k]));
+                p.timer.armed[k] = false;
+            }
+            for (hipEvent_t& e : p.flightBefore) HIP_TRY(hipEventCreate(&e));
+            p.timer.level = timerLevel;
+            p.dw = dw;
+            p.dw.cond0 = p.c0;
+            p.dw.nCond = p.c1 - p.c0;
+            p.dw.chunk0 = hcp[p.c0].chunkBegin;
+            p.dw.nChunks = hcp[p.c1 - 1].chunkBegin + hcp[p.c1 - 1].nChunks - p.dw.chunk0;
+            p.dw.queue = queue.p + i * kFlightClasses * kXcds * kQueueStride;
+            if (nGroups) {
+                p.dw.group0 = hGroup[p.c0];
+                p.dw.nGroups = (p.c1 < nCond ? hGroup[p.c1] : nGroups) - p.dw.group0;
+            }
+            p.dw.planMarks = p.dw.planPairs = 0;
+            for (int c = p.c0; c < p.c1; ++c) {
+                if (hcp[c].nMain > kPlanDirect) p.dw.planMarks = 1;
+                if (hcp[c].nChunks > kPairsDirect) p.dw.planPairs = 1;
+            }
+            p.dh = dh;
+            int first = 0, count = 0;
+            for (const SlotRange& r : hr) {
+                if (r.cond < p.c0) ++first;
+                else if (r.cond < p.c1) ++count;
+            }
+            p.dh.ranges = ranges.p + first;
+            p.dh.nRanges = count;
+        }
         return EKMC_OK;
     }
 
@@ -741,9 +832,9 @@ public:
         tb.maxEnergy = maxEnergy;
         tb.step = maxEnergy / (double)(I - 1);
         HIP_TRY(launch_tables<V>(tsrc, cs[c].N, tb.step, envShift, tables.p + hcp[c].tableOffset, nutot64.p,
-                                 numax64.p, stream));
-        HIP_TRY(hipMemcpyAsync(pinNumax.p, numax64.p, (size_t)I * sizeof(double), hipMemcpyDeviceToHost, stream));
-        HIP_TRY(hipStreamSynchronize(stream));
+                                 numax64.p, cur));
+        HIP_TRY(hipMemcpyAsync(pinNumax.p, numax64.p, (size_t)I * sizeof(double), hipMemcpyDeviceToHost, cur));
+        HIP_TRY(hipStreamSynchronize(cur));
         tb.numax.assign(pinNumax.p, pinNumax.p + I);
         host_add(H_TABLES, ms_since(t0));
         return EKMC_OK;
@@ -771,17 +862,23 @@ public:
         return EKMC_OK;
     }
 
-    // The histogram grid and phase rows for the next kernels, uploaded only
-    // when they differ from the last upload (the stream was synchronized
-    // since that upload, so the pinned staging may be rewritten).
-    ekmc_status upload_hist_grid(const std::vector<double>& g, const std::vector<int32_t>& r) {
-        if (g == upGrid && r == upRow) return EKMC_OK;
-        std::memcpy(pinGrid.p, g.data(), g.size() * sizeof(double));
-        std::memcpy(pinRow.p, r.data(), r.size() * sizeof(int32_t));
-        HIP_TRY(hipMemcpyAsync(grid.p, pinGrid.p, g.size() * sizeof(double), hipMemcpyHostToDevice, stream));
-        HIP_TRY(hipMemcpyAsync(phaseRow.p, pinRow.p, r.size() * sizeof(int32_t), hipMemcpyHostToDevice, stream));
-        upGrid = g;
-        upRow = r;
+    // The histogram grid and phase rows of conditions [c0, c0 + r.size()) for the
+    // next kernels, uploaded only when they differ from the last upload (the
+    // stream was synchronized since that upload, so the pinned staging may be
+    // rewritten).
+    ekmc_status upload_hist_grid(int c0, const std::vector<double>& g, const std::vector<int32_t>& r) {
+        if (upRow.empty()) {
+            upGrid.assign((size_t)nCond * 6, -1.0);
+            upRow.assign(nCond, -2);
+        }
+        if (std::equal(g.begin(), g.end(), upGrid.begin() + 6 * c0) && std::equal(r.begin(), r.end(), upRow.begin() + c0))
+            return EKMC_OK;
+        std::copy(g.begin(), g.end(), pinGrid.p + 6 * c0);
+        std::copy(r.begin(), r.end(), pinRow.p + c0);
+        HIP_TRY(hipMemcpyAsync(grid.p + 6 * c0, pinGrid.p + 6 * c0, g.size() * sizeof(double), hipMemcpyHostToDevice, cur));
+        HIP_TRY(hipMemcpyAsync(phaseRow.p + c0, pinRow.p + c0, r.size() * sizeof(int32_t), hipMemcpyHostToDevice, cur));
+        std::copy(g.begin(), g.end(), upGrid.begin() + 6 * c0);
+        std::copy(r.begin(), r.end(), upRow.begin() + c0);
         return EKMC_OK;
     }
 
@@ -790,42 +887,55 @@ public:
         kstat[K_COUNT + ph].second += ms;
     }
 
-    ekmc_status sync_timers() {
+    // The time of the part's kernels.  Flights of two parts overlap: a part's
+    // count from the end of those counted before, so that the sum is the time
+    // in which flights ran, and an interval counts once.
+    ekmc_status sync_timers(Part& p) {
         for (int k = 0; k < K_COUNT; ++k) {
-            if (!timer.armed[k]) continue;
-            float ms = 0;
-            if (hipEventElapsedTime(&ms, timer.start[k], timer.stop[k]) == hipSuccess) {
-                kstat[k].first += 1;
-                kstat[k].second += ms;
+            if (!p.timer.armed[k]) continue;
+            p.timer.armed[k] = false;
+            float ms = 0, since = 0;
+            if (hipEventElapsedTime(&ms, p.timer.start[k], p.timer.stop[k]) != hipSuccess) continue;
+            if (k == K_ADVANCE && parts.size() > 1) {
+                if (lastFlight && hipEventElapsedTime(&since, lastFlight, p.timer.stop[k]) == hipSuccess)
+                    ms = std::max(0.0f, std::min(ms, since));
+                lastFlight = p.timer.stop[k];
             }
-            timer.armed[k] = false;
+            kstat[k].first += k != K_ADVANCE || p.countsInterval ? 1 : 0;
+            kstat[k].second += ms;
         }
         return EKMC_OK;
     }
 
     // Flight-kernel work lists of the running conditions, per field case.
-    std::vector<int32_t> hlist;
-    ekmc_status rebuild_lists() {
-        std::vector<int32_t> act(nCond);
-        for (int c = 0; c < nCond; ++c) act[c] = cs[c].finished ? 0 : 1;
+    // a condition of [c0, c1) with this field case is running
+    bool runs(int fieldCase, int c0, int c1) const {
+        for (int c = c0; c < c1; ++c)
+            if (!cs[c].finished && cs[c].fieldCase == fieldCase) return true;
+        return false;
+    }
+    ekmc_status rebuild_lists(Part& p) {
+        std::vector<int32_t> act(nCond, 0);
+        for (int c = p.c0; c < p.c1; ++c) act[c] = cs[c].finished ? 0 : 1;
+        std::vector<int32_t>& hlist = p.hlist;
+        FlightLists& fl = p.fl;
+        int32_t* list = flist.p + p.dw.chunk0;  // the part's place in the list buffer
+        // DC and DC+B conditions share one launch when both are running (the
+        // whole batch counts: which kernel flies a condition does not depend on
+        // how the batch is cut)
+        const bool merged = mergeDC && runs(FIELD_DC, 0, nCond) && runs(FIELD_DC_B, 0, nCond);
         // rebuilt when the running set changes, and every 256 intervals for
         // the order (below)
-        if (act == listActive && ++listAge < 256) return EKMC_OK;
-        listAge = 0;
-        listActive = act;
+        if (act == p.listActive && merged == p.listMerged && ++p.listAge < 256) return EKMC_OK;
+        p.listAge = 0;
+        p.listActive = act;
+        p.listMerged = merged;
         hlist.clear();
         fl = FlightLists{};
         const bool thermal = num.gas_temperature_effect != EKMC_GASTEMP_FALSE;
-        // DC and DC+B conditions share one launch when both are running
-        bool anyDC = false, anyDCB = false;
-        for (int c = 0; c < nCond; ++c) {
-            anyDC |= act[c] && cs[c].fieldCase == FIELD_DC;
-            anyDCB |= act[c] && cs[c].fieldCase == FIELD_DC_B;
-        }
-        const bool merged = anyDC && anyDCB && mergeDC;
         for (int fc = 0; fc < kFlightClasses; ++fc) {
             const size_t begin = hlist.size();
-            for (int c = 0; c < nCond; ++c) {
+            for (int c = p.c0; c < p.c1; ++c) {
                 if (!act[c]) continue;
                 const int cls = merged && (cs[c].fieldCase == FIELD_DC || cs[c].fieldCase == FIELD_DC_B) ? FLIGHT_DC_ANY
                                                                                                       : cs[c].fieldCase;
@@ -844,7 +954,7 @@ public:
             const int64_t count = (int64_t)(hlist.size() - begin);
             if (count == 0) continue;
             FlightList& l = fl.cls[fc];
-            l.list = flist.p + begin;
+            l.list = list + begin;
             const int64_t waves = (int64_t)flight_blocks_per_cu<V>(fc, thermal, P, dh) * cus * (kBlock / kWave);
             l.oneShot = count <= waves;
             // parts of equal chunk count (one shot) or of equal expected work
@@ -860,19 +970,20 @@ public:
             int64_t longest = 0;
             for (x = 0; x < kXcds; ++x) longest = std::max<int64_t>(longest, l.part[x + 1] - l.part[x]);
             const int64_t perBlock = kBlock / kWave;
-            fl.grid[fc] = (int32_t)(l.oneShot ? kXcds * ((longest + perBlock - 1) / perBlock) : waves / perBlock);
+            fl.grid[fc] = (int32_t)(l.oneShot ? kXcds * ((longest + perBlock - 1) / perBlock) : waves / perBlock * (parts.size() > 1 ? kPartShare : 8) / 8);
         }
         if (!hlist.empty())
-            HIP_TRY(hipMemcpyAsync(flist.p, hlist.data(), hlist.size() * sizeof(int32_t), hipMemcpyHostToDevice, stream));
-        HIP_TRY(hipStreamSynchronize(stream));
+            HIP_TRY(hipMemcpyAsync(list, hlist.data(), hlist.size() * sizeof(int32_t), hipMemcpyHostToDevice, p.stream));
+        HIP_TRY(hipStreamSynchronize(p.stream));
         return EKMC_OK;
     }
 
     // Fixed-order reduction of the chunk records and the download of the
     // per-condition summaries.
-    hipError_t launch_reduce() {
-        hipError_t e = launch_finish(dw, P, stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(hsum.p, summary.p, hsum.n * sizeof(double), hipMemcpyDeviceToHost, stream);
+    hipError_t launch_reduce(const DevWork& w, hipStream_t st) {
+        hipError_t e = launch_finish(w, P, st);
+        const size_t at = (size_t)w.cond0 * summarySize, n = (size_t)w.nCond * summarySize;
+        if (e == hipSuccess) e = hipMemcpyAsync(hsum.p + at, summary.p + at, n * sizeof(double), hipMemcpyDeviceToHost, st);
         return e;
     }
 
@@ -883,37 +994,37 @@ public:
     // captured once into a HIP graph and replayed.  It holds kernels and one
     // copy only, no memset nodes.  Per-kernel timing (EKMC_KERNEL_TIMING=all)
     // records events between the kernels and runs them one by one.
-    ekmc_status launch_cycle() {
-        if (!useGraph || timer.level >= 2) {
-            HIP_TRY(launch_popctl<V>(ds, dw, stream));
-            HIP_TRY(launch_settle<V>(ds, dw, stream));
-            HIP_TRY(launch_reduce());
+    ekmc_status launch_cycle(Part& p) {
+        if (!useGraph || timerLevel >= 2) {
+            HIP_TRY(launch_popctl<V>(ds, p.dw, p.stream));
+            HIP_TRY(launch_settle<V>(ds, p.dw, p.stream));
+            HIP_TRY(launch_reduce(p.dw, p.stream));
             return EKMC_OK;
         }
-        if (!cycExec) {
-            HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-            hipError_t e = launch_popctl<V>(ds, dw, stream);
-            if (e == hipSuccess) e = launch_settle<V>(ds, dw, stream);
-            if (e == hipSuccess) e = launch_reduce();
+        if (!p.cycExec) {
+            HIP_TRY(hipStreamBeginCapture(p.stream, hipStreamCaptureModeThreadLocal));
+            hipError_t e = launch_popctl<V>(ds, p.dw, p.stream);
+            if (e == hipSuccess) e = launch_settle<V>(ds, p.dw, p.stream);
+            if (e == hipSuccess) e = launch_reduce(p.dw, p.stream);
             hipGraph_t g = nullptr;
-            const hipError_t ec = hipStreamEndCapture(stream, &g);
+            const hipError_t ec = hipStreamEndCapture(p.stream, &g);
             if (e == hipSuccess) e = ec;
             if (e != hipSuccess) {
                 if (g) (void)hipGraphDestroy(g);
                 HIP_TRY(e);
             }
-            cycGraph = g;
-            HIP_TRY(hipGraphInstantiate(&cycExec, cycGraph, nullptr, nullptr, 0));
+            p.cycGraph = g;
+            HIP_TRY(hipGraphInstantiate(&p.cycExec, p.cycGraph, nullptr, nullptr, 0));
         }
-        HIP_TRY(hipGraphLaunch(cycExec, stream));
+        HIP_TRY(hipGraphLaunch(p.cycExec, p.stream));
         return EKMC_OK;
     }
 
-    ekmc_status wait_summary() {
+    ekmc_status wait_summary(Part& p) {
         const auto t0 = Clock::now();
-        HIP_TRY(hipStreamSynchronize(stream));
+        HIP_TRY(hipStreamSynchronize(p.stream));
         host_add(H_WAIT, ms_since(t0));
-        sync_timers();
+        sync_timers(p);
         return EKMC_OK;
     }
 
@@ -965,9 +1076,9 @@ public:
         std::vector<unsigned long long> tmp;
         auto pull = [&](DevBuf<unsigned long long>& b, size_t off, size_t n, std::vector<double>& dst) -> ekmc_status {
             tmp.resize(n);
-            HIP_TRY(hipMemcpyAsync(tmp.data(), b.p + off, n * sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
-            HIP_TRY(hipMemsetAsync(b.p + off, 0, n * sizeof(unsigned long long), stream));
-            HIP_TRY(hipStreamSynchronize(stream));
+            HIP_TRY(hipMemcpyAsync(tmp.data(), b.p + off, n * sizeof(unsigned long long), hipMemcpyDeviceToHost, cur));
+            HIP_TRY(hipMemsetAsync(b.p + off, 0, n * sizeof(unsigned long long), cur));
+            HIP_TRY(hipStreamSynchronize(cur));
             if (dst.size() < n) dst.assign(n, 0.0);
             for (size_t i = 0; i < n; ++i) dst[i] += (double)tmp[i];
             return EKMC_OK;
@@ -1143,11 +1254,11 @@ public:
             hcp[c].tsync = 0;
         }
         HIP_TRY(hipMemcpyAsync(dconds.p, hcp.data(), nCond * sizeof(CondParams), hipMemcpyHostToDevice, stream));
-        set_kernel_timer(&timer);
+        set_kernel_timer(&parts[0].timer);
         HIP_TRY(launch_init<V>(ds, dw, totalMain, mainBase.p, thermalDev.p, stream));
         HIP_TRY(launch_settle<V>(ds, dw, stream));
-        HIP_TRY(launch_reduce());
-        ekmc_status st = wait_summary();
+        HIP_TRY(launch_reduce(dw, stream));
+        ekmc_status st = wait_summary(parts[0]);
         if (st != EKMC_OK) return st;
         for (int c = 0; c < nCond; ++c) {
             Cond& C = cs[c];
@@ -1167,87 +1278,136 @@ public:
     }
 
     // ------------------------------------------------------------------ step
+    // The parts' intervals run one after another in turn: while the host sums up
+    // and prepares one part, the others' kernels run.
     ekmc_status step(int nsync, int* running) override {
         if (!initialized) return fail(EKMC_ERR_STATE, "ekmc_initialize has not been called");
-        set_kernel_timer(&timer);
-        for (int s = 0; s < nsync; ++s) {
-            const auto tPrep = Clock::now();
-            int active = 0;
-            bool anyHist = false, anyHistKernel = false;
-            std::vector<double> hgrid((size_t)nCond * 6, 0.0);
-            std::vector<int32_t> hrow(nCond, -1);
-            for (int c = 0; c < nCond; ++c) {
-                Cond& C = cs[c];
-                hcp[c].active = C.finished ? 0 : 1;
-                double* gr = &hgrid[(size_t)c * 6];
-                gr[0] = C.eedfStep; gr[1] = C.cosStep; gr[2] = C.radStep; gr[3] = C.axStep; gr[4] = C.maxSpeed;
-                if (C.histRequest) {
-                    // a running condition's flight kernel counts the state as it
-                    // loads it (flag 2); a finished one needs the histogram kernel
-                    gr[5] = (C.finished || !fusedHist) ? 1 : 2;
-                    anyHist = true;
-                    anyHistKernel |= C.finished || !fusedHist;
-                    hrow[c] = C.histPhase;
-                    C.histRequest = 0;
-                }
-                if (C.finished) continue;
-                ++active;
-                {
-                    ekmc_status st = check_max_collision_frequency(c);
-                    if (st != EKMC_OK) return st;
-                }
-                double dts = num.sync_time_x_max_coll_freq / C.trial;
-                C.tsync = C.time + dts;
-                ++C.nSync;
-                ++C.syncIndex;
-                hcp[c].trial = C.trial;
-                hcp[c].trialInv = 1.0 / C.trial;
-                hcp[c].tsync = C.tsync;
-                hcp[c].step = C.tab.step;
-                hcp[c].syncIndex = C.syncIndex;
+        ekmc_status st = EKMC_OK;
+        for (int s = 0; s <= nsync && st == EKMC_OK; ++s) {
+            bool first = true;
+            for (Part& p : parts) {
+                cur = p.stream;
+                if (p.inFlight && (st = end_interval(p)) != EKMC_OK) break;
+                if (s == nsync) continue;
+                // the launch of a part that runs only one of DC and DC+B depends
+                // on whether a part after it still runs the other
+                const bool dc = runs(FIELD_DC, p.c0, p.c1), dcb = runs(FIELD_DC_B, p.c0, p.c1);
+                for (Part* q = &p + 1; dc != dcb && q != parts.data() + parts.size() && st == EKMC_OK; ++q)
+                    if (q->inFlight && runs(dc ? FIELD_DC_B : FIELD_DC, q->c0, q->c1)) {
+                        cur = q->stream;
+                        st = end_interval(*q);
+                        cur = p.stream;
+                    }
+                if (st != EKMC_OK) break;
+                if ((st = start_interval(p)) != EKMC_OK) break;
+                p.countsInterval = first;
+                if (p.inFlight) first = false;
             }
-            if (active == 0 && !anyHist) break;
-            {
-                // histograms of the state sampled at the end of the previous interval
-                ekmc_status st = upload_hist_grid(hgrid, hrow);
-                if (st != EKMC_OK) return st;
-                if (anyHistKernel) HIP_TRY(launch_hist<V>(ds, dh, stream));
-            }
-            if (active == 0) { HIP_TRY(hipStreamSynchronize(stream)); break; }
-            {
-                ekmc_status st = rebuild_lists();
-                if (st != EKMC_OK) return st;
-            }
-            host_add(H_PREPARE, ms_since(tPrep));
-            const auto tLaunch = Clock::now();
-            std::memcpy(pinCond.p, hcp.data(), nCond * sizeof(CondParams));
-            HIP_TRY(hipMemcpyAsync(dconds.p, pinCond.p, nCond * sizeof(CondParams), hipMemcpyHostToDevice, stream));
-            HIP_TRY(launch_flights<V>(ds, dw, dpr, tables.p, dh, fl, stream));
-            if (snap && !snap->taken && !cs[snap->cond].finished) {
-                ekmc_status st = take_snapshot(*snap);
-                if (st != EKMC_OK) return st;
-            }
-            ekmc_status st = launch_cycle();
-            if (st != EKMC_OK) return st;
-            host_add(H_LAUNCH, ms_since(tLaunch));
-            if ((st = wait_summary()) != EKMC_OK) return st;
-            const auto tPost = Clock::now();
-            for (int c = 0; c < nCond; ++c) {
-                if (cs[c].finished) continue;
-                st = post_interval(c);
-                if (st != EKMC_OK) return st;
-            }
-            host_add(H_POST, ms_since(tPost));
+            if (first) break;  // nothing runs
         }
+        if (st != EKMC_OK) {  // the error stays; the other parts' intervals are summed up
+            const std::string msg = g_error;
+            for (Part& p : parts) {
+                cur = p.stream;
+                if (p.inFlight) (void)end_interval(p);
+            }
+            g_error = msg;
+        }
+        cur = stream;
+        if (st != EKMC_OK) return st;
         int run = 0;
         for (auto& C : cs) run += C.finished ? 0 : 1;
         if (running) *running = run;
         return EKMC_OK;
     }
 
+    // Launch the next interval of a part, if any of its conditions is running.
+    ekmc_status start_interval(Part& p) {
+        const auto tPrep = Clock::now();
+        set_kernel_timer(&p.timer);
+        const int n = p.c1 - p.c0;
+        int active = 0;
+        bool anyHist = false, anyHistKernel = false;
+        std::vector<double> hgrid((size_t)n * 6, 0.0);
+        std::vector<int32_t> hrow(n, -1);
+        for (int c = p.c0; c < p.c1; ++c) {
+            Cond& C = cs[c];
+            hcp[c].active = C.finished ? 0 : 1;
+            double* gr = &hgrid[(size_t)(c - p.c0) * 6];
+            gr[0] = C.eedfStep; gr[1] = C.cosStep; gr[2] = C.radStep; gr[3] = C.axStep; gr[4] = C.maxSpeed;
+            if (C.histRequest) {
+                // a running condition's flight kernel counts the state as it
+                // loads it (flag 2); a finished one needs the histogram kernel
+                gr[5] = (C.finished || !fusedHist) ? 1 : 2;
+                anyHist = true;
+                anyHistKernel |= C.finished || !fusedHist;
+                hrow[c - p.c0] = C.histPhase;
+                C.histRequest = 0;
+            }
+            if (C.finished) continue;
+            ++active;
+            {
+                ekmc_status st = check_max_collision_frequency(c);
+                if (st != EKMC_OK) return st;
+            }
+            double dts = num.sync_time_x_max_coll_freq / C.trial;
+            C.tsync = C.time + dts;
+            ++C.nSync;
+            ++C.syncIndex;
+            hcp[c].trial = C.trial;
+            hcp[c].trialInv = 1.0 / C.trial;
+            hcp[c].tsync = C.tsync;
+            hcp[c].step = C.tab.step;
+            hcp[c].syncIndex = C.syncIndex;
+        }
+        if (active == 0 && !anyHist) return EKMC_OK;
+        {
+            // histograms of the state sampled at the end of the previous interval
+            ekmc_status st = upload_hist_grid(p.c0, hgrid, hrow);
+            if (st != EKMC_OK) return st;
+            if (anyHistKernel) HIP_TRY(launch_hist<V>(ds, p.dh, p.stream));
+        }
+        if (active == 0) { HIP_TRY(hipStreamSynchronize(p.stream)); return EKMC_OK; }
+        {
+            ekmc_status st = rebuild_lists(p);
+            if (st != EKMC_OK) return st;
+        }
+        host_add(H_PREPARE, ms_since(tPrep));
+        const auto tLaunch = Clock::now();
+        std::copy(hcp.begin() + p.c0, hcp.begin() + p.c1, pinCond.p + p.c0);
+        HIP_TRY(hipMemcpyAsync(dconds.p + p.c0, pinCond.p + p.c0, n * sizeof(CondParams), hipMemcpyHostToDevice, p.stream));
+        std::swap(p.timer.start[K_ADVANCE], p.flightBefore[0]);
+        std::swap(p.timer.stop[K_ADVANCE], p.flightBefore[1]);
+        HIP_TRY(launch_flights<V>(ds, p.dw, dpr, tables.p, p.dh, p.fl, p.stream));
+        if (snap && !snap->taken && snap->cond >= p.c0 && snap->cond < p.c1 && !cs[snap->cond].finished) {
+            ekmc_status st = take_snapshot(*snap, p.stream);
+            if (st != EKMC_OK) return st;
+        }
+        ekmc_status st = launch_cycle(p);
+        if (st != EKMC_OK) return st;
+        p.inFlight = true;
+        host_add(H_LAUNCH, ms_since(tLaunch));
+        return EKMC_OK;
+    }
+
+    // Wait for a part's interval and sum it up.
+    ekmc_status end_interval(Part& p) {
+        p.inFlight = false;
+        ekmc_status st = wait_summary(p);
+        if (st != EKMC_OK) return st;
+        const auto tPost = Clock::now();
+        for (int c = p.c0; c < p.c1; ++c) {
+            if (cs[c].finished) continue;
+            st = post_interval(c);
+            if (st != EKMC_OK) return st;
+        }
+        host_add(H_POST, ms_since(tPost));
+        return EKMC_OK;
+    }
+
     // Every alive electron of condition c's slots (main slots, then the
     // newborn regions of its chunks), in slot order.
-    ekmc_status take_snapshot(PoolSnap& sn) {
+    ekmc_status take_snapshot(PoolSnap& sn, hipStream_t st) {
         const int c = sn.cond;
         const int64_t begin = hcp[c].base, end = c + 1 < nCond ? hcp[c + 1].base : capacity;
         const size_t n = (size_t)(end - begin);
@@ -1255,7 +1415,7 @@ public:
         std::vector<RecA<V>> ha(n);
         std::vector<RecB<V>> hb(split_record<V>() ? n : 0);
         std::vector<uint8_t> al(n);
-        HIP_TRY(hipStreamSynchronize(stream));
+        HIP_TRY(hipStreamSynchronize(st));
         HIP_TRY(hipMemcpy(ha.data(), recA.p + begin, n * sizeof(RecA<V>), hipMemcpyDeviceToHost));
         if (split_record<V>())
             HIP_TRY(hipMemcpy(hb.data(), recB.p + begin, n * sizeof(RecB<V>), hipMemcpyDeviceToHost));
@@ -1368,12 +1528,13 @@ public:
             if (C.histRequest) { gr[5] = 1; any = true; hrow[c] = C.histPhase; C.histRequest = 0; }
         }
         {
-            ekmc_status st = upload_hist_grid(hgrid, hrow);
+            set_kernel_timer(&parts[0].timer);
+            ekmc_status st = upload_hist_grid(0, hgrid, hrow);
             if (st != EKMC_OK) return st;
             if (any) HIP_TRY(launch_hist<V>(ds, dh, stream));
         }
         HIP_TRY(hipStreamSynchronize(stream));
-        sync_timers();
+        sync_timers(parts[0]);
         for (int c = 0; c < nCond; ++c) {
             Cond& C = cs[c];
             if (C.ssTime == kNonDef || C.nIntPts < 50)

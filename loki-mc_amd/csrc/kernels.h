@@ -121,8 +121,10 @@ struct DevWork {
     double* summary;              // [n_cond * summarySize]
     int summarySize;
     int recSize;                  // 3P + 8
-    int nChunks;
-    int nCond;
+    // the launch's part of the batch: chunks, conditions and reduction groups
+    int chunk0, nChunks;
+    int cond0, nCond;
+    int group0;
     // Reduction groups, for batches with a condition of more than
     // kFinishDirect work units: fixed ranges of at most kFinishGroup units
     // of one condition, summed by one block each before the per-condition
@@ -134,7 +136,7 @@ struct DevWork {
     const int32_t* condGroups;    // [n_cond] groups of the condition
     double* tailG;                // [nGroups * CT_SIZE]
     double* momG;                 // [nGroups * kMomentRecord]
-    int nGroups;
+    int nGroups;                  // of the launch's part
 };
 // A block of k_finish sums 28 records at a time; for a condition of more than
 // 448 work units (16 turns) a group kernel, with about as many groups as units

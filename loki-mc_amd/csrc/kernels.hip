@@ -952,8 +952,8 @@ __host__ __device__ __forceinline__ bool plans_direct(const CondParams& cp) { re
 // added to the condition's total.
 __global__ __launch_bounds__(kBlock) void k_marks(const uint8_t* alive, DevWork w) {
     const int lane = lane_id();
-    const int cid = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (cid >= w.nChunks) return;
+    const int cid = w.chunk0 + blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+    if (cid >= w.chunk0 + w.nChunks) return;
     const Chunk ch = w.chunks[cid];
     const int sur = w.surplusC[cid];
     const CondParams& cp = w.conds[ch.cond];
@@ -1129,7 +1129,7 @@ __device__ void removal_threshold(const CondParams& cp, int64_t K, PopPlan& pl, 
 __global__ __launch_bounds__(1024) void k_plan_marks(DevWork w) {
     __shared__ int64_t lds[2 * kWave + 1];
     __shared__ PopLds L;
-    const int c = blockIdx.x;
+    const int c = w.cond0 + blockIdx.x;
     const CondParams cp = w.conds[c];
     if (!cp.active || plans_direct(cp)) return;
     PopPlan pl = plan_of(pop_total(w, c), cp);
@@ -1196,8 +1196,8 @@ __global__ __launch_bounds__(kBlock) void k_apply_marks(DevState<V> s, DevWork w
     __shared__ PopLds L;
     __shared__ int conds[kWavesPerBlock];
     const int lane = lane_id(), wid = threadIdx.x / kWave;
-    const int cid = blockIdx.x * kWavesPerBlock + wid;
-    const bool in = cid < w.nChunks;
+    const int cid = w.chunk0 + blockIdx.x * kWavesPerBlock + wid;
+    const bool in = cid < w.chunk0 + w.nChunks;
     Chunk ch = {};
     int c = -1, sur = 0, holes = 0, mine = 0;
     PopPlan pl = {};
@@ -1248,7 +1248,7 @@ __global__ __launch_bounds__(kBlock) void k_apply_marks(DevState<V> s, DevWork w
 // others in the per-chunk counts.)
 __global__ __launch_bounds__(1024) void k_plan_pairs(DevWork w) {
     __shared__ int64_t lds[2 * kWave + 1];
-    const int c = blockIdx.x;
+    const int c = w.cond0 + blockIdx.x;
     const CondParams cp = w.conds[c];
     if (!cp.active || cp.nChunks <= kPairsDirect) return;
     const CondPop pop = pop_total(w, c);
@@ -1378,8 +1378,8 @@ __device__ __forceinline__ double wave_sums(const double (&m)[kMomentRecord], in
 template <typename V>
 __global__ __launch_bounds__(kBlock) void k_settle(DevState<V> s, DevWork w) {
     const int lane = lane_id();
-    const int cid = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (cid >= w.nChunks) return;
+    const int cid = w.chunk0 + blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+    if (cid >= w.chunk0 + w.nChunks) return;
     const Chunk me = w.chunks[cid];
     const CondParams& cp = w.conds[me.cond];
     if (!cp.active) return;
@@ -1557,7 +1557,7 @@ __global__ __launch_bounds__(kBlock) void k_hist(DevState<V> s, const SlotRange*
 // field f of records r, r + kFinishRows, ... in order (neighbouring threads
 // read neighbouring fields), then thread f adds the rows.  The integer
 // accumulators are converted and cleared for the next interval, and block 0
-// resets the flight-kernel work queues.
+// resets the flight-kernel work queues of the launch's part.
 constexpr int kFinishFields = CT_SIZE + kMomentRecord;
 constexpr int kFinishBlock = 1024;
 constexpr int kFinishRows = kFinishBlock / (kFinishFields + 1);
@@ -1600,7 +1600,7 @@ __device__ double finish_reduce(const double* tsrc, const double* msrc, size_t f
 // record layout of the chunk tails and moments.
 __global__ __launch_bounds__(kFinishBlock) void k_finish_group(DevWork w) {
     __shared__ double red[kFinishRows][kFinishFields + 1];
-    const int g = blockIdx.x;
+    const int g = w.group0 + blockIdx.x;
     if (!w.conds[w.groupCond[g]].active) return;
     const double tot = finish_reduce(w.tailC, w.momC, (size_t)w.groupFirst[g], w.groupCount[g], red);
     if (threadIdx.x < kFinishFields) {
@@ -1612,8 +1612,8 @@ __global__ __launch_bounds__(kFinishBlock) void k_finish_group(DevWork w) {
 
 __global__ __launch_bounds__(kFinishBlock) void k_finish(DevWork w, int P) {
     __shared__ double red[kFinishRows][kFinishFields + 1];
-    const int c = blockIdx.x;
-    if (c == 0)
+    const int c = w.cond0 + blockIdx.x;
+    if (blockIdx.x == 0)
         for (int k = threadIdx.x; k < kFlightClasses * kXcds; k += blockDim.x) w.queue[k * kQueueStride] = 0;
     const CondParams cp = w.conds[c];
     if (!cp.active) return;

@@ -270,7 +270,7 @@ public:
     DevBuf<Chunk> chunks;
     DevBuf<int32_t> holesC, surplusC, markC, flist, phaseRow, cylFlag;
     DevBuf<int64_t> holeOff, surOff, markOff, mainBase;
-    DevBuf<double> tailC, momC, summary, thermalDev, grid;
+    DevBuf<double> tailC, momC, thermalDev, grid;
     DevBuf<int32_t> gCond, gFirst, gCount, cGroup, cGroups;  // reduction groups (huge conditions)
     DevBuf<double> tailG, momG;
     int nGroups = 0;
@@ -297,8 +297,8 @@ public:
     int nCells = 1000, nCos = 100, nRad = 200, nAx = 200, nPhases = 0;
     int n3 = 0;  // cells per axis of the 3D EVDF (0: none)
     bool anyCyl = false, anyAC = false;
-    PinnedBuf<double> hsum;         // per-condition summaries of the last interval
-    PinnedBuf<CondParams> pinCond;  // staging of the per-interval condition upload
+    PinnedBuf<double> hsum;         // per-condition summaries of the last interval, written by k_finish
+    PinnedBuf<CondParams> pinCond;  // the interval's condition parameters, read by the flight kernel
     PinnedBuf<double> pinNumax;     // running maximum frequency of a rebuilt table
     DevBuf<double> tsrcD, nutot64, numax64;
     DevBuf<int> tsrcI;
@@ -353,7 +353,7 @@ public:
         alive.release(); tables.release(); dconds.release(); chunks.release(); holesC.release();
         surplusC.release(); markC.release(); flist.release(); phaseRow.release(); cylFlag.release();
         holeOff.release(); surOff.release(); markOff.release(); mainBase.release(); tailC.release();
-        momC.release(); summary.release(); thermalDev.release(); grid.release(); accCount.release();
+        momC.release(); thermalDev.release(); grid.release(); accCount.release();
         gCond.release(); gFirst.release(); gCount.release(); cGroup.release(); cGroups.release();
         tailG.release(); momG.release();
         accGain.release(); accLoss.release(); plans.release(); prec.release(); iproc.release(); dproc.release();
@@ -560,6 +560,9 @@ public:
         HIP_TRY(hipMemsetAsync(pop.p, 0, pop.n * sizeof(CondPop), stream));
         recSize = event_record_size(P);
         summarySize = recSize + kMomentRecord + 8;
+        HIP_TRY(hsum.alloc((size_t)n * summarySize));
+        std::memset(hsum.p, 0, hsum.n * sizeof(double));
+        dw.summary = hsum.p;
         HIP_TRY(tailC.alloc((size_t)nChunks * CT_SIZE));
         HIP_TRY(momC.alloc((size_t)nChunks * kMomentRecord));
         HIP_TRY(hipMemsetAsync(tailC.p, 0, (size_t)nChunks * CT_SIZE * sizeof(double), stream));
@@ -593,7 +596,6 @@ public:
                 HIP_TRY(hipStreamSynchronize(stream));
             }
         }
-        HIP_TRY(summary.alloc((size_t)n * summarySize));
         HIP_TRY(accCount.alloc((size_t)n * P)); HIP_TRY(accGain.alloc((size_t)n * P)); HIP_TRY(accLoss.alloc((size_t)n * P));
         HIP_TRY(hipMemsetAsync(accCount.p, 0, (size_t)n * P * 8, stream));
         HIP_TRY(hipMemsetAsync(accGain.p, 0, (size_t)n * P * 8, stream));
@@ -700,7 +702,7 @@ public:
         dw.markC = markC.p; dw.holeOff = holeOff.p; dw.surOff = surOff.p; dw.markOff = markOff.p;
         dw.holeList = holeList.p; dw.laneMarks = laneMarks.p; dw.pop = pop.p; dw.tailC = tailC.p; dw.momC = momC.p; dw.accCount = accCount.p;
         dw.accGain = accGain.p; dw.accLoss = accLoss.p; dw.plans = plans.p;
-        dw.status = status.p; dw.queue = queue.p; dw.summary = summary.p; dw.summarySize = summarySize;
+        dw.status = status.p; dw.queue = queue.p; dw.summarySize = summarySize;
         dw.recSize = recSize; dw.chunk0 = 0; dw.nChunks = nChunks; dw.cond0 = 0; dw.nCond = n; dw.group0 = 0;
         dw.groupCond = gCond.p; dw.groupFirst = gFirst.p; dw.groupCount = gCount.p;
         dw.condGroup = cGroup.p; dw.condGroups = cGroups.p; dw.tailG = tailG.p; dw.momG = momG.p;
@@ -739,8 +741,6 @@ public:
         HIP_TRY(thermalDev.alloc(n));
         HIP_TRY(hipMemcpyAsync(mainBase.p, mb.data(), n * sizeof(int64_t), hipMemcpyHostToDevice, stream));
         HIP_TRY(hipMemcpyAsync(thermalDev.p, td.data(), n * sizeof(double), hipMemcpyHostToDevice, stream));
-        HIP_TRY(hsum.alloc((size_t)n * summarySize));
-        std::memset(hsum.p, 0, hsum.n * sizeof(double));
         HIP_TRY(pinCond.alloc(n));
         HIP_TRY(pinGrid.alloc((size_t)n * 6));
         HIP_TRY(pinRow.alloc(n));
@@ -784,12 +784,13 @@ public:
                 p.stream = nullptr;
                 HIP_TRY(hipStreamCreateWithFlags(&p.stream, hipStreamNonBlocking));
             }
+            // times only: nothing waits on them for memory
             for (int k = 0; k < K_COUNT; ++k) {
-                HIP_TRY(hipEventCreate(&p.timer.start[k]));
-                HIP_TRY(hipEventCreate(&p.timer.stop[k]));
+                HIP_TRY(hipEventCreateWithFlags(&p.timer.start[k], hipEventReleaseToDevice));
+                HIP_TRY(hipEventCreateWithFlags(&p.timer.stop[k], hipEventReleaseToDevice));
                 p.timer.armed[k] = false;
             }
-            for (hipEvent_t& e : p.flightBefore) HIP_TRY(hipEventCreate(&e));
+            for (hipEvent_t& e : p.flightBefore) HIP_TRY(hipEventCreateWithFlags(&e, hipEventReleaseToDevice));
             p.timer.level = timerLevel;
             p.dw = dw;
             p.dw.cond0 = p.c0;
@@ -978,34 +979,25 @@ public:
         return EKMC_OK;
     }
 
-    // Fixed-order reduction of the chunk records and the download of the
-    // per-condition summaries.
-    hipError_t launch_reduce(const DevWork& w, hipStream_t st) {
-        hipError_t e = launch_finish(w, P, st);
-        const size_t at = (size_t)w.cond0 * summarySize, n = (size_t)w.nCond * summarySize;
-        if (e == hipSuccess) e = hipMemcpyAsync(hsum.p + at, summary.p + at, n * sizeof(double), hipMemcpyDeviceToHost, st);
-        return e;
-    }
-
     // The cycle that follows the flights -- population control, sampling,
-    // the reduction and the summary download -- is the same launches with the
+    // the reduction into the host's summary -- is the same launches with the
     // same arguments every interval (the device state and work descriptors
     // are fixed at creation; what changes lives in device memory), so it is
-    // captured once into a HIP graph and replayed.  It holds kernels and one
-    // copy only, no memset nodes.  Per-kernel timing (EKMC_KERNEL_TIMING=all)
+    // captured once into a HIP graph and replayed.  It holds kernels
+    // only, no memset nodes.  Per-kernel timing (EKMC_KERNEL_TIMING=all)
     // records events between the kernels and runs them one by one.
     ekmc_status launch_cycle(Part& p) {
         if (!useGraph || timerLevel >= 2) {
             HIP_TRY(launch_popctl<V>(ds, p.dw, p.stream));
             HIP_TRY(launch_settle<V>(ds, p.dw, p.stream));
-            HIP_TRY(launch_reduce(p.dw, p.stream));
+            HIP_TRY(launch_finish(p.dw, P, p.stream));
             return EKMC_OK;
         }
         if (!p.cycExec) {
             HIP_TRY(hipStreamBeginCapture(p.stream, hipStreamCaptureModeThreadLocal));
             hipError_t e = launch_popctl<V>(ds, p.dw, p.stream);
             if (e == hipSuccess) e = launch_settle<V>(ds, p.dw, p.stream);
-            if (e == hipSuccess) e = launch_reduce(p.dw, p.stream);
+            if (e == hipSuccess) e = launch_finish(p.dw, P, p.stream);
             hipGraph_t g = nullptr;
             const hipError_t ec = hipStreamEndCapture(p.stream, &g);
             if (e == hipSuccess) e = ec;
@@ -1257,7 +1249,7 @@ public:
         set_kernel_timer(&parts[0].timer);
         HIP_TRY(launch_init<V>(ds, dw, totalMain, mainBase.p, thermalDev.p, stream));
         HIP_TRY(launch_settle<V>(ds, dw, stream));
-        HIP_TRY(launch_reduce(dw, stream));
+        HIP_TRY(launch_finish(dw, P, stream));
         ekmc_status st = wait_summary(parts[0]);
         if (st != EKMC_OK) return st;
         for (int c = 0; c < nCond; ++c) {
@@ -1375,10 +1367,9 @@ public:
         host_add(H_PREPARE, ms_since(tPrep));
         const auto tLaunch = Clock::now();
         std::copy(hcp.begin() + p.c0, hcp.begin() + p.c1, pinCond.p + p.c0);
-        HIP_TRY(hipMemcpyAsync(dconds.p + p.c0, pinCond.p + p.c0, n * sizeof(CondParams), hipMemcpyHostToDevice, p.stream));
         std::swap(p.timer.start[K_ADVANCE], p.flightBefore[0]);
         std::swap(p.timer.stop[K_ADVANCE], p.flightBefore[1]);
-        HIP_TRY(launch_flights<V>(ds, p.dw, dpr, tables.p, p.dh, p.fl, p.stream));
+        HIP_TRY(launch_flights<V>(ds, p.dw, pinCond.p, dpr, tables.p, p.dh, p.fl, p.stream));
         if (snap && !snap->taken && snap->cond >= p.c0 && snap->cond < p.c1 && !cs[snap->cond].finished) {
             ekmc_status st = take_snapshot(*snap, p.stream);
             if (st != EKMC_OK) return st;

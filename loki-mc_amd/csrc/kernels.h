@@ -97,7 +97,7 @@ constexpr int kPopCopies = 8;
 
 // Device work buffers shared by the interval kernels.
 struct DevWork {
-    const CondParams* conds;      // [n_cond]
+    CondParams* conds;            // [n_cond]
     const Chunk* chunks;          // [n_chunks]
     int32_t* holesC;              // [n_chunks] holes left after the chunk's own refill
     int32_t* surplusC;            // [n_chunks] newborns left in the chunk's region
@@ -118,7 +118,7 @@ struct DevWork {
     PopPlan* plans;               // [n_cond]
     uint32_t* status;             // [n_cond]
     uint32_t* queue;              // [kFlightClasses * kXcds * kQueueStride] work-queue counters of the flight kernels
-    double* summary;              // [n_cond * summarySize]
+    double* summary;              // [n_cond * summarySize], pinned host memory
     int summarySize;
     int recSize;                  // 3P + 8
     // the launch's part of the batch: chunks, conditions and reduction groups
@@ -229,9 +229,11 @@ inline int64_t table_block_size(int I, int P, int G) { return (int64_t)I * (2 * 
 template <typename V>
 hipError_t launch_init(const DevState<V>& s, const DevWork& w, int64_t totalMain,
                        const int64_t* mainBase, const double* thermalDev, hipStream_t st);
-// The flights of one interval: one launch per flight class with work.
+// The flights of one interval: one launch per flight class with work.  `conds`
+// are the conditions' parameters in pinned host memory; the flights write them to
+// w.conds for the kernels that follow.
 template <typename V>
-hipError_t launch_flights(const DevState<V>& s, const DevWork& w, const DevProcesses& pr,
+hipError_t launch_flights(const DevState<V>& s, const DevWork& w, const CondParams* conds, const DevProcesses& pr,
                           const V* tables, const DevHist& h, const FlightLists& fl, hipStream_t st);
 // Removals after the flights: the same launches every interval.
 template <typename V>

@@ -564,15 +564,15 @@ __device__ __forceinline__ void hist_count(const DevHist& h, int c, const double
 // passes of BoltzmannMC.C:630-681 for this set of electrons).
 template <typename V, int FC, bool THERMAL, int HIST>
 __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWork& w, const DevProcesses& pr,
-                                              const V* tables, const DevHist& h, int cid, unsigned long long* cnt,
-                                              lds_uint4* ring, bool lines) {
+                                              const V* tables, const DevHist& h, const CondParams* conds, int cid,
+                                              unsigned long long* cnt, lds_uint4* ring, bool lines) {
     const int lane = lane_id();
     const int P = pr.P;
     long long* gainL = (long long*)(cnt + P);
     long long* lossL = gainL + P;
     const Chunk ch = w.chunks[cid];
     const int c = ch.cond;
-    const CondParams cp = w.conds[c];
+    const CondParams cp = conds[c];
     const int64_t I = cp.I;
     const V* cumul = tables + cp.tableOffset;
     const V* interp = cumul + I * P;
@@ -834,7 +834,7 @@ template <typename V, int FC> constexpr int flight_waves_per_eu() { return sizeo
 // and EVDF 146 -> 126 us, one condition of 9.5e5 in FP64 155 -> 148 us, 24 AC
 // conditions of 2e5 557 -> 523 us; no difference for the 64-condition scan.)
 template <typename V, int FC, bool THERMAL, int HIST>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_waves_per_eu<V, FC>()))) void k_advance(DevState<V> s, DevWork w, DevProcesses pr, const V* tables,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_waves_per_eu<V, FC>()))) void k_advance(DevState<V> s, DevWork w, const CondParams* conds, DevProcesses pr, const V* tables,
                                                     DevHist h, FlightList fl, uint32_t* queue) {
     extern __shared__ unsigned char smem[];
     constexpr int kRingWave = ring_segs<V>() * rec_pieces<V>() * kRingSeg;  // 16-byte pieces per wave
@@ -845,6 +845,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_w
     uint4* procL = (uint4*)smem;
     for (int i = threadIdx.x; i < pr.P * (int)(sizeof(ProcRec) / 16); i += kBlock)
         procL[i] = ((const uint4*)pr.proc)[i];
+    // The interval's parameters are read where the host wrote them, and written to
+    // w.conds for the kernels that follow; k_finish writes the summaries to host
+    // memory in turn.  A copy either way cost a launch and its gap: passes of one
+    // condition of 1e4 electrons (64 intervals) 5.90 -> 5.47 ms, of 1e5 in FP64 7.99 ->
+    // 7.52, of 9.5e5 (32) 6.40 -> 6.17; no difference for 1.6e7 electrons and more.
+    static_assert(sizeof(CondParams) % 8 == 0, "whole words");
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < w.nCond * (int)(sizeof(CondParams) / 8); i += gridDim.x * kBlock)
+        ((uint64_t*)(w.conds + w.cond0))[i] = ((const uint64_t*)(conds + w.cond0))[i];
     __syncthreads();
     DevProcesses prl = pr;
     prl.proc = (const ProcRec*)smem;
@@ -862,7 +870,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_w
             if (fl.oneShot || x == xcd) break;
             continue;
         }
-        advance_chunk<V, FC, THERMAL, HIST>(s, w, prl, tables, h, fl.list[item], cnt, ring, !fl.oneShot);
+        advance_chunk<V, FC, THERMAL, HIST>(s, w, prl, tables, h, conds, fl.list[item], cnt, ring, !fl.oneShot);
         if (fl.oneShot) break;
     }
 }
@@ -1875,30 +1883,30 @@ static const void* flight_kernel(int hist) {
 }
 
 template <typename V, int FC, bool TH, int HIST>
-static void launch_advance_hist(const DevState<V>& s, const DevWork& w, const DevProcesses& pr, const V* tables,
+static void launch_advance_hist(const DevState<V>& s, const DevWork& w, const CondParams* conds, const DevProcesses& pr, const V* tables,
                                 const DevHist& h, const FlightLists& fl, hipStream_t st) {
     dim3 g(fl.grid[FC]), b(kBlock);
     const size_t lds = flight_lds<V>(pr.P, h.histLds);
-    hipLaunchKernelGGL((k_advance<V, FC, TH, HIST>), g, b, lds, st, s, w, pr, tables, h, fl.cls[FC],
+    hipLaunchKernelGGL((k_advance<V, FC, TH, HIST>), g, b, lds, st, s, w, conds, pr, tables, h, fl.cls[FC],
                        w.queue + FC * kXcds * kQueueStride);
 }
 
 template <typename V, int FC, bool TH>
-static void launch_advance_th(const DevState<V>& s, const DevWork& w, const DevProcesses& pr, const V* tables,
+static void launch_advance_th(const DevState<V>& s, const DevWork& w, const CondParams* conds, const DevProcesses& pr, const V* tables,
                               const DevHist& h, const FlightLists& fl, hipStream_t st) {
     switch (hist_mode(h)) {
-        case HIST_LDS: launch_advance_hist<V, FC, TH, HIST_LDS>(s, w, pr, tables, h, fl, st); break;
-        case HIST_LDS_CYL: launch_advance_hist<V, FC, TH, HIST_LDS_CYL>(s, w, pr, tables, h, fl, st); break;
-        default: launch_advance_hist<V, FC, TH, HIST_HBM>(s, w, pr, tables, h, fl, st); break;
+        case HIST_LDS: launch_advance_hist<V, FC, TH, HIST_LDS>(s, w, conds, pr, tables, h, fl, st); break;
+        case HIST_LDS_CYL: launch_advance_hist<V, FC, TH, HIST_LDS_CYL>(s, w, conds, pr, tables, h, fl, st); break;
+        default: launch_advance_hist<V, FC, TH, HIST_HBM>(s, w, conds, pr, tables, h, fl, st); break;
     }
 }
 
 template <typename V, int FC>
-static void launch_advance_case(const DevState<V>& s, const DevWork& w, const DevProcesses& pr, const V* tables,
+static void launch_advance_case(const DevState<V>& s, const DevWork& w, const CondParams* conds, const DevProcesses& pr, const V* tables,
                                 const DevHist& h, const FlightLists& fl, hipStream_t st) {
     if (fl.grid[FC] == 0) return;
-    if (pr.gasTempEffect == 0) launch_advance_th<V, FC, false>(s, w, pr, tables, h, fl, st);
-    else launch_advance_th<V, FC, true>(s, w, pr, tables, h, fl, st);
+    if (pr.gasTempEffect == 0) launch_advance_th<V, FC, false>(s, w, conds, pr, tables, h, fl, st);
+    else launch_advance_th<V, FC, true>(s, w, conds, pr, tables, h, fl, st);
 }
 
 template <typename V>
@@ -1926,15 +1934,15 @@ int flight_blocks_per_cu(int fc, bool thermal, int P, const DevHist& h) {
 }
 
 template <typename V>
-hipError_t launch_flights(const DevState<V>& s, const DevWork& w, const DevProcesses& pr, const V* tables,
+hipError_t launch_flights(const DevState<V>& s, const DevWork& w, const CondParams* conds, const DevProcesses& pr, const V* tables,
                           const DevHist& h, const FlightLists& fl, hipStream_t st) {
     timer_start(K_ADVANCE, st);
-    launch_advance_case<V, FIELD_DC>(s, w, pr, tables, h, fl, st);
-    launch_advance_case<V, FIELD_AC>(s, w, pr, tables, h, fl, st);
-    launch_advance_case<V, FIELD_DC_B>(s, w, pr, tables, h, fl, st);
-    launch_advance_case<V, FIELD_ECR>(s, w, pr, tables, h, fl, st);
-    launch_advance_case<V, FIELD_AC_B>(s, w, pr, tables, h, fl, st);
-    launch_advance_case<V, FLIGHT_DC_ANY>(s, w, pr, tables, h, fl, st);
+    launch_advance_case<V, FIELD_DC>(s, w, conds, pr, tables, h, fl, st);
+    launch_advance_case<V, FIELD_AC>(s, w, conds, pr, tables, h, fl, st);
+    launch_advance_case<V, FIELD_DC_B>(s, w, conds, pr, tables, h, fl, st);
+    launch_advance_case<V, FIELD_ECR>(s, w, conds, pr, tables, h, fl, st);
+    launch_advance_case<V, FIELD_AC_B>(s, w, conds, pr, tables, h, fl, st);
+    launch_advance_case<V, FLIGHT_DC_ANY>(s, w, conds, pr, tables, h, fl, st);
     timer_stop(K_ADVANCE, st);
     return hipGetLastError();
 }
@@ -2008,7 +2016,7 @@ hipError_t launch_op_philox(int64_t n, const uint32_t* ctr, const uint32_t* key,
 #define EKMC_INSTANTIATE(V)                                                                                   \
     template hipError_t launch_init<V>(const DevState<V>&, const DevWork&, int64_t, const int64_t*,           \
                                        const double*, hipStream_t);                                           \
-    template hipError_t launch_flights<V>(const DevState<V>&, const DevWork&, const DevProcesses&, const V*,  \
+    template hipError_t launch_flights<V>(const DevState<V>&, const DevWork&, const CondParams*, const DevProcesses&, const V*,  \
                                           const DevHist&, const FlightLists&, hipStream_t);                   \
     template hipError_t launch_popctl<V>(const DevState<V>&, const DevWork&, hipStream_t);                    \
     template hipError_t launch_settle<V>(const DevState<V>&, const DevWork&, hipStream_t);                    \

@@ -66,6 +66,33 @@ struct DevProcesses {
     const double* gasFrac;   // [G]
 };
 
+// Division by a value known beforehand, with the result an IEEE division gives:
+// hi is 1 / d rounded, lo the rest of 1 / d, q = x hi + x lo within one ulp of
+// x / d, and by Markstein's theorem (IBM J. Res. Dev. 34, 1990) fma(r, hi, q) with
+// the exact residual r = x - q d is x / d rounded.  (Results below 2^-969 and
+// infinite x excepted.)
+// Four instructions for the eleven dependent ones of a division; an FP64 flight
+// made five divisions by the charge, the trial frequency, the table step and the
+// cyclotron frequency.  With sine and cosine taken together, flight kernel per
+// interval in FP64: one condition of 3e7 electrons 2304 -> 2106 us, the
+// 64-condition scan 1484 -> 1423, one condition of 1e5 69.3 -> 66.5, four ECR
+// conditions 89 -> 75.
+struct Reciprocal {
+    double hi, lo;
+};
+inline Reciprocal reciprocal(double d) {
+    const double hi = 1.0 / d;
+    return {hi, __builtin_fma(-hi, d, 1.0) * hi};
+}
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline double divide(double x, double d, const Reciprocal& r) {
+    const double q = __builtin_fma(x, r.hi, x * r.lo);
+    return __builtin_fma(__builtin_fma(-q, d, x), r.hi, q);
+}
+constexpr Reciprocal kChargeInv = {6.241509125883258e+18, -290.37367373329124};
+
 // One working condition as the kernels see it.
 struct CondParams {
     // fields (BoltzmannMC.C:453-489)
@@ -89,6 +116,8 @@ struct CondParams {
     // per interval
     double trial;            // trial collision frequency [1/s]
     double trialInv;         // 1 / trial
+    Reciprocal trialRec, stepRec, nRec, cycRec;  // of trial, step, N and cyclotron
+    double vEx, az;          // e E_x / (m_e W), e E_z / m_e
     double tsync;            // synchronization time of this interval [s]
     double step;             // table energy step [eV]
     uint64_t seed;           // Philox key of this condition

@@ -126,7 +126,9 @@ template <> __device__ __forceinline__ float EventRng<float>::u(int s) {
 
 // Free time -ln(U)/nu_trial (BoltzmannMC.C:652-653): FP64 in the reference
 // order; FP32 with the hardware logarithm and the reciprocal frequency.
-__device__ __forceinline__ double free_time(double u, const CondParams& c) { return -log(u) / c.trial; }
+__device__ __forceinline__ double free_time(double u, const CondParams& c) {
+    return divide(-log(u), c.trial, c.trialRec);
+}
 __device__ __forceinline__ float free_time(float u, const CondParams& c) {
     return -__logf(u) * (float)c.trialInv;
 }
@@ -135,7 +137,7 @@ __device__ __forceinline__ float free_time(float u, const CondParams& c) {
 // FP32 with the hardware sine/cosine, whose argument is in turns.
 __device__ __forceinline__ void turn_sincos(double u, double& s, double& co) {
     const double a = (2.0 * kPi) * u;
-    s = sin(a); co = cos(a);
+    sincos(a, &s, &co);
 }
 __device__ __forceinline__ void turn_sincos(float u, float& s, float& co) {
     s = __builtin_amdgcn_sinf(u); co = __builtin_amdgcn_cosf(u);
@@ -159,7 +161,7 @@ template <typename V> __device__ __forceinline__ V sqr_norm(V a, V b, V c) {
 // electron energy [eV] of a velocity, 0.5*m_e*|v|^2/e in the reference order
 __device__ __forceinline__ double energy_of(double vx, double vy, double vz) {
 #pragma clang fp contract(off)
-    return 0.5 * kMass * sqr_norm(vx, vy, vz) / kCharge;
+    return divide(0.5 * kMass * sqr_norm(vx, vy, vz), kCharge, kChargeInv);
 }
 __device__ __forceinline__ float energy_of(float vx, float vy, float vz) {
 #pragma clang fp contract(off)
@@ -204,9 +206,10 @@ __device__ inline void flight(const CondParams& c, Electron<double>& e, double d
         } break;
         case FIELD_AC: {
             double w = c.omega, phi = w * e.t;
-            double sinPhi = sin(phi), cosPhi = cos(phi);
+            double sinPhi, cosPhi, sinPhase, cosPhase;
+            sincos(phi, &sinPhi, &cosPhi);
             double wDt = w * dt, phase = wDt + phi;
-            double sinPhase = sin(phase), cosPhase = cos(phase);
+            sincos(phase, &sinPhase, &cosPhase);
             double e_me_w = q / (me * w);
             double aux1 = e_me_w / w * (cosPhase + wDt * sinPhi - cosPhi);
             double aux2 = e_me_w * (sinPhi - sinPhase);
@@ -218,9 +221,10 @@ __device__ inline void flight(const CondParams& c, Electron<double>& e, double d
         } break;
         case FIELD_DC_B: {
             double W = c.cyclotron, WDt = W * dt;
-            double sW = sin(WDt), cW = cos(WDt);
-            double sW_W = sW / W, aux2 = (cW - 1.0) / W;
-            double vEx = q * c.E[0] / (me * W), az = q * c.E[2] / me;
+            double sW, cW;
+            sincos(WDt, &sW, &cW);
+            double sW_W = divide(sW, W, c.cycRec), aux2 = divide(cW - 1.0, W, c.cycRec);
+            double vEx = c.vEx, az = c.az;
             e.x += v0 * sW_W + (v1 + vEx) * aux2;
             e.y += -v0 * aux2 + v1 * sW_W + vEx * (sW_W - dt);
             e.z += v2 * dt - 0.5 * az * dt * dt;
@@ -230,30 +234,37 @@ __device__ inline void flight(const CondParams& c, Electron<double>& e, double d
         } break;
         case FIELD_ECR: {
             double W = c.cyclotron, phi = W * e.t;
-            double sinPhi = sin(phi), cosPhi = cos(phi);
-            double WDt = W * dt, sW = sin(WDt), cW = cos(WDt);
-            double phase = WDt + phi, sinPhase = sin(phase), cosPhase = cos(phase);
+            double sinPhi, cosPhi, sW, cW, sinPhase, cosPhase;
+            sincos(phi, &sinPhi, &cosPhi);
+            double WDt = W * dt;
+            sincos(WDt, &sW, &cW);
+            double phase = WDt + phi;
+            sincos(phase, &sinPhase, &cosPhase);
             double cosOpp = cos(phi - WDt);
             double e_me_W = q / (me * W);
             double vEx = e_me_W * c.E[0], vEz = e_me_W * c.E[2];
-            double sW_W = sW / W, cWm1_W = (cW - 1.0) / W, cosPhase_W = cosPhase / W;
-            e.x += v0 * sW_W + v1 * cWm1_W - 0.25 * vEx * (cosPhase_W - cosOpp / W + 2.0 * dt * sinPhase);
+            double sW_W = divide(sW, W, c.cycRec), cWm1_W = divide(cW - 1.0, W, c.cycRec), cosPhase_W = divide(cosPhase, W, c.cycRec);
+            e.x += v0 * sW_W + v1 * cWm1_W - 0.25 * vEx * (cosPhase_W - divide(cosOpp, W, c.cycRec) + 2.0 * dt * sinPhase);
             e.y += -v0 * cWm1_W + v1 * sW_W + 0.5 * vEx * (dt * cosPhase_W - 2.0 * cWm1_W * sinPhi - cosPhi * sW_W);
-            e.z += v2 * dt + vEz * (cosPhase_W - cosPhi / W + dt * sinPhi);
+            e.z += v2 * dt + vEz * (cosPhase_W - divide(cosPhi, W, c.cycRec) + dt * sinPhi);
             e.vx = v0 * cW - v1 * sW - 0.5 * vEx * (WDt * cosPhase + cosPhi * sW);
             e.vy = v0 * sW + v1 * cW - 0.5 * vEx * (WDt * cW * sinPhi + (WDt * cosPhi - sinPhi) * sW);
             e.vz = v2 + vEz * (sinPhi - sinPhase);
         } break;
         default: {
             double w = c.omega, W = c.cyclotron, phi = w * e.t;
-            double sinPhi = sin(phi), cosPhi = cos(phi);
-            double wDt = w * dt, swD = sin(wDt), cwD = cos(wDt);
-            double phase = wDt + phi, sinPhase = sin(phase), cosPhase = cos(phase);
-            double WDt = W * dt, sW = sin(WDt), cW = cos(WDt);
+            double sinPhi, cosPhi, swD, cwD, sinPhase, cosPhase, sW, cW;
+            sincos(phi, &sinPhi, &cosPhi);
+            double wDt = w * dt;
+            sincos(wDt, &swD, &cwD);
+            double phase = wDt + phi;
+            sincos(phase, &sinPhase, &cosPhase);
+            double WDt = W * dt;
+            sincos(WDt, &sW, &cW);
             double w2 = w * w, W2 = W * W, d = w2 - W2;
             double vEx = q / (me * W) * c.E[0], vEz = q / (me * w) * c.E[2];
             double vEx_d = vEx / d, WvEx_d = W * vEx_d;
-            double sW_W = sW / W, cWm1_W = (cW - 1.0) / W, wSinPhi = w * sinPhi;
+            double sW_W = divide(sW, W, c.cycRec), cWm1_W = divide(cW - 1.0, W, c.cycRec), wSinPhi = w * sinPhi;
             e.x += v0 * sW_W + v1 * cWm1_W + WvEx_d * (cosPhi * (cwD - cW) + (wSinPhi * sW_W - sinPhi * swD));
             e.y += -v0 * cWm1_W + v1 * sW_W - vEx_d / w * ((W2 + w2 * cW - w2) * sinPhi + W2 * (w * cosPhi * sW_W - sinPhase));
             e.z += v2 * dt + vEz * ((cosPhase - cosPhi) / w + dt * sinPhi);
@@ -466,9 +477,13 @@ template <typename V> struct ColdRow {
     int k1, k2;
     V w1, w2;
 };
+__device__ __forceinline__ double in_steps(double eps, const CondParams& c) { return divide(eps, c.step, c.stepRec); }
+__device__ __forceinline__ float in_steps(float eps, const CondParams& c) { return eps / (float)c.step; }
+__device__ __forceinline__ double per_density(double f, const CondParams& c) { return divide(f, c.N, c.nRec); }
+__device__ __forceinline__ float per_density(float f, const CondParams& c) { return f / (float)c.N; }
 template <typename V> __device__ __forceinline__ ColdRow<V> cold_row(const CondParams& c, const Electron<V>& e) {
     ColdRow<V> r;
-    const V over = e.eps / (V)c.step;
+    const V over = in_steps(e.eps, c);
     r.k1 = (int)fmin(over, (V)(c.I - 1));
     r.k2 = (int)fmin((V)(r.k1 + 1), (V)(c.I - 1));
     r.w1 = (V)r.k2 - over;
@@ -525,7 +540,7 @@ __device__ __forceinline__ int cold_choose(const CondParams& c, const DevProcess
     const V* i1 = interp + (size_t)r.k1 * P;
     const V* i2 = interp + (size_t)r.k2 * P;
     const V speed = sqrt(sqr_norm(e.vx, e.vy, e.vz));
-    const V randCS = randF / (V)c.N / speed;
+    const V randCS = per_density(randF, c) / speed;
     return channel_search(c1, c2, i1, i2, r.w1, r.w2, 0, P - 1, randCS, (V)0, (V)0, speed, false);
 }
 
@@ -552,7 +567,7 @@ __device__ __forceinline__ int thermal_choose(const CondParams& c, const DevProc
     turn_sincos(r4, s4, c4r);
     V aux1 = sqrt((V)-2 * log_of(r1));
     V vers[3] = {aux1 * c2r, aux1 * s2, sqrt((V)-2 * log_of(r3)) * c4r};
-    V randCS = e.nue * r5 / (V)c.N;
+    V randCS = per_density(e.nue * r5, c);
     V prevSum = (V)0, rel = (V)0, sd = (V)0;
     int row = -1, L = 0, R = 0;
     constexpr int kBatch = 4;

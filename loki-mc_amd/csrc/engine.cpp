@@ -508,6 +508,12 @@ public:
             cp.freq = cs[c].omega / (2.0 * kPi);
             cp.I = I;
             cp.N = cs[c].N;
+            cp.nRec = reciprocal(cp.N);
+            if (cs[c].cyc != 0) {
+                cp.cycRec = reciprocal(cs[c].cyc);
+                cp.vEx = kCharge * cs[c].E[0] / (kMass * cs[c].cyc);
+            }
+            cp.az = kCharge * cs[c].E[2] / kMass;
             cp.gasEnergy = cs[c].gasEnergy;
             cp.seed = num.seed ^ ((uint64_t)c * 0x9E3779B97F4A7C15ull);
             cp.tableOffset = (int64_t)c * table_block_size(I, P, pl.G);
@@ -1348,8 +1354,10 @@ public:
             ++C.syncIndex;
             hcp[c].trial = C.trial;
             hcp[c].trialInv = 1.0 / C.trial;
+            hcp[c].trialRec = reciprocal(C.trial);
             hcp[c].tsync = C.tsync;
             hcp[c].step = C.tab.step;
+            hcp[c].stepRec = reciprocal(C.tab.step);
             hcp[c].syncIndex = C.syncIndex;
         }
         if (active == 0 && !anyHist) return EKMC_OK;
@@ -1634,6 +1642,7 @@ public:
                            int32_t* pid, double* ejv, double* eje, double* de, void* stage) {
         CondParams cp = hcp[c];
         cp.step = cs[c].tab.step;
+        cp.stepRec = reciprocal(cp.step);
         double *dV = (double*)stage, *dE = dV + 3 * n, *dN = dE + n, *dVar = dN + n, *dEjv = dVar + 11 * n,
                *dEje = dEjv + 3 * n, *dDe = dEje + n;
         int32_t* dpp = (int32_t*)(dDe + n);

@@ -52,8 +52,8 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 // kernel: a null event costs a flight and a null test, not a whole step of
 // the wave's bookkeeping.  Measured per interval on the 64-condition scan,
 // mixed form: 1 / 2 / 3 / 4 events, 0.981 / 0.963 / 0.989 / 1.062 ms (longer
-// runs leave more lanes idle in the loop than they save); FP64 form, whose
-// second flight spills registers: 1 / 2 events, 1.596 / 1.663 ms.
+// runs leave more lanes idle in the loop than they save); FP64 form: 1 / 2
+// events, 1.596 / 1.663 ms.
 template <typename V> constexpr int null_run() { return sizeof(V) == 8 ? 1 : 2; }
 
 // LDS of one wave of the flight kernel: collision tallies [3P] (64-bit), the
@@ -812,15 +812,13 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
     wave_lds_sync();
 }
 
-// Waves per SIMD the flight kernel is compiled for.  FP64: 256 registers per
-// lane, two waves; left to itself the compiler takes 290 (256 VGPRs and 34
-// AGPRs), one wave per SIMD, and the few VGPRs spilled at two waves cost less
-// than the latency one wave cannot hide (measured 2.27 -> 1.60 ms per
-// interval on the 64-condition scan in FP64).  Mixed form: the compiler's
-// choice (150-166 VGPRs, three waves, for the FP32 flight formulas); asking
-// for three waves explicitly gave the same occupancy and a slower schedule
-// (0.962 -> 1.000 ms), asking for four (with a two-segment record ring to
-// fit the LDS) spilled 33-41 VGPRs and ran at 1.062 ms.
+// Waves per SIMD the flight kernel is compiled for.  FP64: two (172-187 VGPRs;
+// its record rings leave the LDS room for two blocks per CU anyway).  Mixed form:
+// the compiler's choice (136-168 VGPRs, three waves).  More waves do not make
+// either faster: with a ring of 80 records and an FP32 envelope, so that the LDS
+// held them, one condition of 3e7 electrons took 2416 us per interval with three
+// FP64 waves against 2354 with two, and 1515 with four mixed waves against 1389
+// with three.
 template <typename V, int FC> constexpr int flight_waves_per_eu() { return sizeof(V) == 8 ? 2 : 1; }
 
 // Flight kernel of one field case.  The work list has one part per XCD

@@ -375,13 +375,16 @@ __device__ __forceinline__ V cos_chi(const DevProcesses& pr, int p, V energy, V 
     return (V)1 - (V)2 * R;      // isotropic
 }
 
-// sin(chi) of a sampled cos(chi).  A sampler can round past 1: the FP32
-// screened-Coulomb quotient (sp + 1 - (2 sp + 1) R) / (sp + 1 - R) at R = 0 is
-// x / x, which an FP32 division of a few ulp need not make 1; that is a
-// scattering angle of 0, not a negative square.
-template <typename V> __device__ __forceinline__ V sin_chi(V cosChi) {
-    return sqrt(fmax((V)1 - cosChi * cosChi, (V)0));
+// A sampled cos(chi) within [-1, 1] (a NaN stays one).  A sampler can round past
+// 1: by a few ulp the FP32 screened-Coulomb quotient (sp + 1 - (2 sp + 1) R) /
+// (sp + 1 - R) at R = 0, x / x in a division that need not make it 1; by far more
+// the Surendra quotient (2 + e - 2 (1 + e)^R) / e, whose numerator cancels (in FP32
+// 1.4e-3 at 1e-5 eV).  Past 1 is a scattering angle of 0: its sine would be the root
+// of a negative number, and a direction with a longer cosine adds energy.
+template <typename V> __device__ __forceinline__ V cosine(V c) {
+    return c > (V)1 ? (V)1 : (c < (V)-1 ? (V)-1 : c);
 }
+template <typename V> __device__ __forceinline__ V sin_chi(V cosChi) { return sqrt((V)1 - cosChi * cosChi); }
 
 template <typename V> struct Sph { V norm, sinT, cosT, sinP, cosP; };
 
@@ -662,6 +665,7 @@ __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron
     V cc;
     if (boeuf) cc = sqrt(scE / net);
     else cc = cos_chi<V>(pr, chosen, (V)before, scE, rng, 6);
+    cc = cosine(cc);
     const V sc = sin_chi(cc);
     V se, ce;
     turn_sincos(rng.u(7), se, ce);
@@ -695,10 +699,10 @@ __device__ __forceinline__ void apply_collision(const DevProcesses& pr, Electron
     // the ejected electron (ionizationCollision, BoltzmannMC.C:1228-1267)
     V cCe, sCe, sEe, cEe;
     if (boeuf) {
-        cCe = sqrt(ej / net); sCe = sin_chi(cCe);
+        cCe = cosine(sqrt(ej / net)); sCe = sin_chi(cCe);
         sEe = -se; cEe = -ce;
     } else {
-        cCe = cos_chi<V>(pr, chosen, inc, ej, rng, 9);
+        cCe = cosine(cos_chi<V>(pr, chosen, inc, ej, rng, 9));
         sCe = sin_chi(cCe);
         turn_sincos(rng.u(10), sEe, cEe);
     }

@@ -745,9 +745,10 @@ __device__ inline void collide(const CondParams& c, const DevProcesses& pr, cons
 // call 0 of the electron's current event), fly to t_sync or to the collision
 // and, in the cold branch, run the null test.  Phase B: the channel choice
 // and collision operator of a real (or thermal) collision.
-// An electron at t_sync (a collision or an ejection exactly there) flies for no
-// time, which changes nothing, and keeps its pending or undefined free time.
-// Every lane runs the same instructions to the end: what differs between a
+// An electron at t_sync (a collision or an ejection exactly there) is done as it
+// is: a flight of no time would still leave the roundings of its formulas in the
+// position and of the energy in the field gain.
+// Every other lane runs the same instructions to the end: what differs between a
 // flight that ends at t_sync and one that ends in a null or a real collision is
 // selected, not branched on.  (The step's flights are the largest part of a
 // wave's time, 44 % on the 64-condition scan, and a third of their instructions
@@ -760,16 +761,18 @@ template <typename V, int FC, bool THERMAL>
 __device__ __forceinline__ int step_a(const CondParams& c, const DevProcesses& pr, const V* nutot, const V* envHi,
                                       const V* envLo, Electron<V>& e, EventRng<V>& rng, bool& escape,
                                       double& gain) {
+    escape = false;
+    gain = 0;
+    if (e.t == c.tsync) return STEP_DONE;
     // the draws of every lane, whether it needs a free time, a variate of the
     // null test or neither (a pending flight that outlasts the interval)
     rng.prime0();
     const V fresh = free_time(rng.u(0), c);
-    const bool idle = e.t == c.tsync;
-    const bool draw = e.tfree < (V)0 && !idle;  // pending free time undefined (NON_DEF is negative)
+    const bool draw = e.tfree < (V)0;  // pending free time undefined (NON_DEF is negative)
     e.tfree = draw ? fresh : e.tfree;
     e.nue = draw ? (V)c.trial : e.nue;
     // one flight for both outcomes (a wave holds both kinds of lanes)
-    const bool partial = idle || e.t + (double)e.tfree > c.tsync;
+    const bool partial = e.t + (double)e.tfree > c.tsync;
     const double dt = partial ? c.tsync - e.t : (double)e.tfree;
     if (FC == FLIGHT_DC_ANY) {
         if (c.fieldCase == FIELD_DC) flight<FIELD_DC>(c, e, dt, gain);

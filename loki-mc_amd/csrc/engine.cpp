@@ -336,7 +336,6 @@ public:
 
     ~Engine() override {
         if (stream) (void)hipStreamSynchronize(stream);
-        set_kernel_timer(nullptr);
         for (Part& p : parts) {
             if (p.stream) (void)hipStreamSynchronize(p.stream);
             if (p.cycExec) (void)hipGraphExecDestroy(p.cycExec);
@@ -994,16 +993,16 @@ public:
     // records events between the kernels and runs them one by one.
     ekmc_status launch_cycle(Part& p) {
         if (!useGraph || timerLevel >= 2) {
-            HIP_TRY(launch_popctl<V>(ds, p.dw, p.stream));
-            HIP_TRY(launch_settle<V>(ds, p.dw, p.stream));
-            HIP_TRY(launch_finish(p.dw, P, p.stream));
+            HIP_TRY(launch_popctl<V>(ds, p.dw, &p.timer, p.stream));
+            HIP_TRY(launch_settle<V>(ds, p.dw, &p.timer, p.stream));
+            HIP_TRY(launch_finish(p.dw, P, &p.timer, p.stream));
             return EKMC_OK;
         }
         if (!p.cycExec) {
             HIP_TRY(hipStreamBeginCapture(p.stream, hipStreamCaptureModeThreadLocal));
-            hipError_t e = launch_popctl<V>(ds, p.dw, p.stream);
-            if (e == hipSuccess) e = launch_settle<V>(ds, p.dw, p.stream);
-            if (e == hipSuccess) e = launch_finish(p.dw, P, p.stream);
+            hipError_t e = launch_popctl<V>(ds, p.dw, &p.timer, p.stream);
+            if (e == hipSuccess) e = launch_settle<V>(ds, p.dw, &p.timer, p.stream);
+            if (e == hipSuccess) e = launch_finish(p.dw, P, &p.timer, p.stream);
             hipGraph_t g = nullptr;
             const hipError_t ec = hipStreamEndCapture(p.stream, &g);
             if (e == hipSuccess) e = ec;
@@ -1252,10 +1251,10 @@ public:
             hcp[c].tsync = 0;
         }
         HIP_TRY(hipMemcpyAsync(dconds.p, hcp.data(), nCond * sizeof(CondParams), hipMemcpyHostToDevice, stream));
-        set_kernel_timer(&parts[0].timer);
-        HIP_TRY(launch_init<V>(ds, dw, totalMain, mainBase.p, thermalDev.p, stream));
-        HIP_TRY(launch_settle<V>(ds, dw, stream));
-        HIP_TRY(launch_finish(dw, P, stream));
+        KernelTimer* timer = &parts[0].timer;
+        HIP_TRY(launch_init<V>(ds, dw, totalMain, mainBase.p, thermalDev.p, timer, stream));
+        HIP_TRY(launch_settle<V>(ds, dw, timer, stream));
+        HIP_TRY(launch_finish(dw, P, timer, stream));
         ekmc_status st = wait_summary(parts[0]);
         if (st != EKMC_OK) return st;
         for (int c = 0; c < nCond; ++c) {
@@ -1322,7 +1321,6 @@ public:
     // Launch the next interval of a part, if any of its conditions is running.
     ekmc_status start_interval(Part& p) {
         const auto tPrep = Clock::now();
-        set_kernel_timer(&p.timer);
         const int n = p.c1 - p.c0;
         int active = 0;
         bool anyHist = false, anyHistKernel = false;
@@ -1365,7 +1363,7 @@ public:
             // histograms of the state sampled at the end of the previous interval
             ekmc_status st = upload_hist_grid(p.c0, hgrid, hrow);
             if (st != EKMC_OK) return st;
-            if (anyHistKernel) HIP_TRY(launch_hist<V>(ds, p.dh, p.stream));
+            if (anyHistKernel) HIP_TRY(launch_hist<V>(ds, p.dh, &p.timer, p.stream));
         }
         if (active == 0) { HIP_TRY(hipStreamSynchronize(p.stream)); return EKMC_OK; }
         {
@@ -1377,7 +1375,7 @@ public:
         std::copy(hcp.begin() + p.c0, hcp.begin() + p.c1, pinCond.p + p.c0);
         std::swap(p.timer.start[K_ADVANCE], p.flightBefore[0]);
         std::swap(p.timer.stop[K_ADVANCE], p.flightBefore[1]);
-        HIP_TRY(launch_flights<V>(ds, p.dw, pinCond.p, dpr, tables.p, p.dh, p.fl, p.stream));
+        HIP_TRY(launch_flights<V>(ds, p.dw, pinCond.p, dpr, tables.p, p.dh, p.fl, &p.timer, p.stream));
         if (snap && !snap->taken && snap->cond >= p.c0 && snap->cond < p.c1 && !cs[snap->cond].finished) {
             ekmc_status st = take_snapshot(*snap, p.stream);
             if (st != EKMC_OK) return st;
@@ -1527,10 +1525,9 @@ public:
             if (C.histRequest) { gr[5] = 1; any = true; hrow[c] = C.histPhase; C.histRequest = 0; }
         }
         {
-            set_kernel_timer(&parts[0].timer);
             ekmc_status st = upload_hist_grid(0, hgrid, hrow);
             if (st != EKMC_OK) return st;
-            if (any) HIP_TRY(launch_hist<V>(ds, dh, stream));
+            if (any) HIP_TRY(launch_hist<V>(ds, dh, &parts[0].timer, stream));
         }
         HIP_TRY(hipStreamSynchronize(stream));
         sync_timers(parts[0]);

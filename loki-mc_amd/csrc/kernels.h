@@ -225,25 +225,36 @@ hipError_t launch_tables(const DevTableSrc& src, double N, double step, int envS
 // Elements of one condition's table block.
 inline int64_t table_block_size(int I, int P, int G) { return (int64_t)I * (2 * P + 1 + G) + 2 * kEnvBins; }
 
+// kernel names for timing (index matches the event slots used by the engine)
+enum KernelId { K_INIT = 0, K_ADVANCE, K_MARKS, K_APPLY, K_SETTLE, K_HIST, K_REDUCE, K_COUNT };
+extern const char* kKernelNames[K_COUNT];
+// Per-kernel HIP events, recorded by the launchers that get one (null: none).  Each
+// part of an engine's batch has its own: engines run on several threads at once.
+struct KernelTimer {
+    hipEvent_t start[K_COUNT], stop[K_COUNT];
+    bool armed[K_COUNT];
+    int level;  // 0 none, 1 flight kernels, 2 every kernel
+};
+
 // mainBase[c]: index of condition c's first electron among all main electrons
 template <typename V>
 hipError_t launch_init(const DevState<V>& s, const DevWork& w, int64_t totalMain,
-                       const int64_t* mainBase, const double* thermalDev, hipStream_t st);
+                       const int64_t* mainBase, const double* thermalDev, KernelTimer* timer, hipStream_t st);
 // The flights of one interval: one launch per flight class with work.  `conds`
 // are the conditions' parameters in pinned host memory; the flights write them to
 // w.conds for the kernels that follow.
 template <typename V>
 hipError_t launch_flights(const DevState<V>& s, const DevWork& w, const CondParams* conds, const DevProcesses& pr,
-                          const V* tables, const DevHist& h, const FlightLists& fl, hipStream_t st);
+                          const V* tables, const DevHist& h, const FlightLists& fl, KernelTimer* timer, hipStream_t st);
 // Removals after the flights: the same launches every interval.
 template <typename V>
-hipError_t launch_popctl(const DevState<V>& s, const DevWork& w, hipStream_t st);
+hipError_t launch_popctl(const DevState<V>& s, const DevWork& w, KernelTimer* timer, hipStream_t st);
 // Pairs, clones and the ensemble sums.
 template <typename V>
-hipError_t launch_settle(const DevState<V>& s, const DevWork& w, hipStream_t st);
+hipError_t launch_settle(const DevState<V>& s, const DevWork& w, KernelTimer* timer, hipStream_t st);
 template <typename V>
-hipError_t launch_hist(const DevState<V>& s, const DevHist& h, hipStream_t st);
-hipError_t launch_finish(const DevWork& w, int P, hipStream_t st);
+hipError_t launch_hist(const DevState<V>& s, const DevHist& h, KernelTimer* timer, hipStream_t st);
+hipError_t launch_finish(const DevWork& w, int P, KernelTimer* timer, hipStream_t st);
 // Resident blocks per CU of the flight kernel of field case (or class) fc.
 // (histogram configuration h: the EEDF in LDS when h.histLds >= h.nCells)
 template <typename V>
@@ -267,16 +278,5 @@ hipError_t launch_op_collide(const CondParams* cond, const DevProcesses& pr, con
                              int32_t* pid, double* ejv, double* eje, double* de, hipStream_t st);
 hipError_t launch_op_philox(int64_t n, const uint32_t* ctr, const uint32_t* key, uint32_t* out,
                             hipStream_t st);
-
-// kernel names for timing (index matches the event slots used by the engine)
-enum KernelId { K_INIT = 0, K_ADVANCE, K_MARKS, K_APPLY, K_SETTLE, K_HIST, K_REDUCE, K_COUNT };
-extern const char* kKernelNames[K_COUNT];
-// Per-kernel HIP events recorded by the launchers when set.
-struct KernelTimer {
-    hipEvent_t start[K_COUNT], stop[K_COUNT];
-    bool armed[K_COUNT];
-    int level;  // 0 none, 1 flight kernels, 2 every kernel
-};
-void set_kernel_timer(KernelTimer* t);
 
 }  // namespace ekmc

@@ -33,16 +33,13 @@ namespace ekmc {
 
 const char* kKernelNames[K_COUNT] = {"init", "advance", "marks", "apply_marks", "settle", "hist", "finish"};
 
-static KernelTimer* g_timer = nullptr;
-void set_kernel_timer(KernelTimer* t) { g_timer = t; }
-
 // level 1 times the flight kernels only, level 2 every kernel
-static inline bool timed(int k) { return g_timer && (g_timer->level >= 2 || (g_timer->level == 1 && k == K_ADVANCE)); }
-static inline void timer_start(int k, hipStream_t st) {
-    if (timed(k)) { (void)hipEventRecord(g_timer->start[k], st); }
+static inline bool timed(const KernelTimer* t, int k) { return t && (t->level >= 2 || (t->level == 1 && k == K_ADVANCE)); }
+static inline void timer_start(KernelTimer* t, int k, hipStream_t st) {
+    if (timed(t, k)) (void)hipEventRecord(t->start[k], st);
 }
-static inline void timer_stop(int k, hipStream_t st) {
-    if (timed(k)) { (void)hipEventRecord(g_timer->stop[k], st); g_timer->armed[k] = true; }
+static inline void timer_stop(KernelTimer* t, int k, hipStream_t st) {
+    if (timed(t, k)) { (void)hipEventRecord(t->stop[k], st); t->armed[k] = true; }
 }
 
 constexpr double kFix = 16777216.0;  // 2^24: fixed-point scale of energy sums [eV]
@@ -1871,12 +1868,12 @@ template <typename V> static inline size_t flight_lds(int P, int histLds) {
 
 template <typename V>
 hipError_t launch_init(const DevState<V>& s, const DevWork& w, int64_t totalMain, const int64_t* mainBase,
-                       const double* thermalDev, hipStream_t st) {
+                       const double* thermalDev, KernelTimer* timer, hipStream_t st) {
     if (totalMain == 0) return hipSuccess;
-    timer_start(K_INIT, st);
+    timer_start(timer, K_INIT, st);
     hipLaunchKernelGGL(k_init<V>, dim3(grid_of(totalMain)), dim3(kBlock), 0, st, s, w.conds, w.nCond, totalMain,
                        mainBase, thermalDev);
-    timer_stop(K_INIT, st);
+    timer_stop(timer, K_INIT, st);
     return hipGetLastError();
 }
 
@@ -1948,56 +1945,56 @@ int flight_blocks_per_cu(int fc, bool thermal, int P, const DevHist& h) {
 
 template <typename V>
 hipError_t launch_flights(const DevState<V>& s, const DevWork& w, const CondParams* conds, const DevProcesses& pr, const V* tables,
-                          const DevHist& h, const FlightLists& fl, hipStream_t st) {
-    timer_start(K_ADVANCE, st);
+                          const DevHist& h, const FlightLists& fl, KernelTimer* timer, hipStream_t st) {
+    timer_start(timer, K_ADVANCE, st);
     launch_advance_case<V, FIELD_DC>(s, w, conds, pr, tables, h, fl, st);
     launch_advance_case<V, FIELD_AC>(s, w, conds, pr, tables, h, fl, st);
     launch_advance_case<V, FIELD_DC_B>(s, w, conds, pr, tables, h, fl, st);
     launch_advance_case<V, FIELD_ECR>(s, w, conds, pr, tables, h, fl, st);
     launch_advance_case<V, FIELD_AC_B>(s, w, conds, pr, tables, h, fl, st);
     launch_advance_case<V, FLIGHT_DC_ANY>(s, w, conds, pr, tables, h, fl, st);
-    timer_stop(K_ADVANCE, st);
+    timer_stop(timer, K_ADVANCE, st);
     return hipGetLastError();
 }
 
 template <typename V>
-hipError_t launch_popctl(const DevState<V>& s, const DevWork& w, hipStream_t st) {
+hipError_t launch_popctl(const DevState<V>& s, const DevWork& w, KernelTimer* timer, hipStream_t st) {
     const dim3 g(chunk_grid(w.nChunks)), b(kBlock);
-    timer_start(K_MARKS, st);
+    timer_start(timer, K_MARKS, st);
     hipLaunchKernelGGL(k_marks, g, b, 0, st, s.alive, w);
     if (w.planMarks) hipLaunchKernelGGL(k_plan_marks, dim3(w.nCond), dim3(kPlanBlock), 0, st, w);
-    timer_stop(K_MARKS, st);
-    timer_start(K_APPLY, st);
+    timer_stop(timer, K_MARKS, st);
+    timer_start(timer, K_APPLY, st);
     hipLaunchKernelGGL(k_apply_marks<V>, g, b, 0, st, s, w);
     if (w.planPairs) hipLaunchKernelGGL(k_plan_pairs, dim3(w.nCond), dim3(1024), 0, st, w);
-    timer_stop(K_APPLY, st);
+    timer_stop(timer, K_APPLY, st);
     return hipGetLastError();
 }
 
 template <typename V>
-hipError_t launch_settle(const DevState<V>& s, const DevWork& w, hipStream_t st) {
-    timer_start(K_SETTLE, st);
+hipError_t launch_settle(const DevState<V>& s, const DevWork& w, KernelTimer* timer, hipStream_t st) {
+    timer_start(timer, K_SETTLE, st);
     hipLaunchKernelGGL(k_settle<V>, dim3(chunk_grid(w.nChunks)), dim3(kBlock), 0, st, s, w);
-    timer_stop(K_SETTLE, st);
+    timer_stop(timer, K_SETTLE, st);
     return hipGetLastError();
 }
 
 template <typename V>
-hipError_t launch_hist(const DevState<V>& s, const DevHist& h, hipStream_t st) {
+hipError_t launch_hist(const DevState<V>& s, const DevHist& h, KernelTimer* timer, hipStream_t st) {
     if (h.nRanges == 0) return hipSuccess;
     const int ldsCells = h.nCells <= 8192 ? h.nCells : 0;
     const size_t lds = (size_t)ldsCells * 4;
-    timer_start(K_HIST, st);
+    timer_start(timer, K_HIST, st);
     hipLaunchKernelGGL(k_hist<V>, dim3(h.nRanges), dim3(kBlock), lds, st, s, h.ranges, h, ldsCells);
-    timer_stop(K_HIST, st);
+    timer_stop(timer, K_HIST, st);
     return hipGetLastError();
 }
 
-hipError_t launch_finish(const DevWork& w, int P, hipStream_t st) {
-    timer_start(K_REDUCE, st);
+hipError_t launch_finish(const DevWork& w, int P, KernelTimer* timer, hipStream_t st) {
+    timer_start(timer, K_REDUCE, st);
     if (w.nGroups) hipLaunchKernelGGL(k_finish_group, dim3(w.nGroups), dim3(kFinishBlock), 0, st, w);
     hipLaunchKernelGGL(k_finish, dim3(w.nCond), dim3(kFinishBlock), 0, st, w, P);
-    timer_stop(K_REDUCE, st);
+    timer_stop(timer, K_REDUCE, st);
     return hipGetLastError();
 }
 
@@ -2028,12 +2025,12 @@ hipError_t launch_op_philox(int64_t n, const uint32_t* ctr, const uint32_t* key,
 
 #define EKMC_INSTANTIATE(V)                                                                                   \
     template hipError_t launch_init<V>(const DevState<V>&, const DevWork&, int64_t, const int64_t*,           \
-                                       const double*, hipStream_t);                                           \
+                                       const double*, KernelTimer*, hipStream_t);                                           \
     template hipError_t launch_flights<V>(const DevState<V>&, const DevWork&, const CondParams*, const DevProcesses&, const V*,  \
-                                          const DevHist&, const FlightLists&, hipStream_t);                   \
-    template hipError_t launch_popctl<V>(const DevState<V>&, const DevWork&, hipStream_t);                    \
-    template hipError_t launch_settle<V>(const DevState<V>&, const DevWork&, hipStream_t);                    \
-    template hipError_t launch_hist<V>(const DevState<V>&, const DevHist&, hipStream_t);                     \
+                                          const DevHist&, const FlightLists&, KernelTimer*, hipStream_t);                   \
+    template hipError_t launch_popctl<V>(const DevState<V>&, const DevWork&, KernelTimer*, hipStream_t);                    \
+    template hipError_t launch_settle<V>(const DevState<V>&, const DevWork&, KernelTimer*, hipStream_t);                    \
+    template hipError_t launch_hist<V>(const DevState<V>&, const DevHist&, KernelTimer*, hipStream_t);                     \
     template int flight_blocks_per_cu<V>(int, bool, int, const DevHist&);                                                \
     template hipError_t launch_tables<V>(const DevTableSrc&, double, double, int, V*, double*, double*,        \
                                          hipStream_t);                                                       \

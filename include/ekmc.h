@@ -161,7 +161,8 @@ typedef struct {
     int32_t max_sync_points;                 /* safety cap on sampling points, 0 = none */
     uint64_t seed;                           /* Philox key */
     int32_t work_chunk;                      /* electrons per wavefront work unit (at most
-                                                65535); 0: 1024 for batches above 3.1 M
+                                                65535; taken in whole waves of 64, 65472
+                                                at most); 0: 1024 for batches above 3.1 M
                                                 electrons, else the batch over the resident
                                                 waves, at least 256 */
     int32_t park_lanes;                      /* lanes of a wavefront that wait for a real

@@ -15,6 +15,7 @@ constexpr int kBlock = 256;            // threads per block of every grid-wide k
 constexpr int kWave = 64;              // CDNA wavefront
 constexpr int kChunkDefault = 1024;    // main electrons per wave work unit (64 lanes x 16)
 constexpr int kChunkMin = 256;         // smallest default work unit (small batches)
+constexpr int kChunkMax = 65535 / kWave * kWave;  // whole waves, as many as the 16-bit EEDF counts of a unit hold
 constexpr uint32_t kMaxLoopPerSync = 1u << 22;  // flight cap per electron per interval
 constexpr int kEnvBins = 256;          // bins of the null-test envelope of the total frequency
 

@@ -478,7 +478,7 @@ public:
                               ? kChunkDefault
                               : std::max<int64_t>(kChunkMin, (total + waves - 1) / waves);
         }
-        chunkTarget = std::max<int64_t>(kWave, (chunkTarget + kWave - 1) / kWave * kWave);
+        chunkTarget = std::min<int64_t>(kChunkMax, std::max<int64_t>(kWave, (chunkTarget + kWave - 1) / kWave * kWave));
         envShift = 0;  // envelope bins of 2^envShift table rows, at most kEnvBins of them
         while (((I - 1) >> envShift) >= kEnvBins) ++envShift;
         envShift += num.env_coarsen;

@@ -136,11 +136,8 @@ struct CondParams {
 
 // Per-condition population-control plan, written by device planning kernels.
 struct PopPlan {
-    int64_t holes;       // unfilled main slots after the local refill
-    int64_t surplus;     // newborns still in regions
     int64_t alive;       // M
     int64_t remove;      // R = max(0, M - N)
-    int64_t marks;       // K
     int64_t thrIndex;    // removal threshold: mark j goes iff (key_j, j) <= (thrKey, thrIndex)
     double markProb;     // p
     uint32_t status;

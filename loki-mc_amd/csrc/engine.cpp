@@ -564,7 +564,7 @@ public:
         HIP_TRY(pop.alloc((size_t)kPopCopies * dw.popStride));
         HIP_TRY(hipMemsetAsync(pop.p, 0, pop.n * sizeof(CondPop), stream));
         recSize = event_record_size(P);
-        summarySize = recSize + kMomentRecord + 8;
+        summarySize = recSize + kMomentRecord + 1;
         HIP_TRY(hsum.alloc((size_t)n * summarySize));
         std::memset(hsum.p, 0, hsum.n * sizeof(double));
         dw.summary = hsum.p;
@@ -1441,8 +1441,7 @@ public:
         Cond& C = cs[c];
         const double* ev = &hsum[(size_t)c * summarySize];
         const double* m = ev + recSize;
-        const double* tail = m + kMomentRecord;
-        uint32_t stbits = (uint32_t)tail[6];
+        uint32_t stbits = (uint32_t)m[kMomentRecord];
         if (stbits & ST_ZERO_VELOCITY) return fail(EKMC_ERR_ZERO_VELOCITY, "Trying to use the function 'cart2sph' for a vector with null norm!");
         if (stbits & ST_REGION_OVERFLOW) return fail(EKMC_ERR_CAPACITY, "newborn region of a thread overflowed");
         if (stbits & ST_POPCTL) return fail(EKMC_ERR_CAPACITY, "population control could not draw an exact sample");

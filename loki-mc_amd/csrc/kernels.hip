@@ -903,8 +903,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(flight_w
 __device__ __forceinline__ PopPlan plan_of(const CondPop& pop, const CondParams& cp) {
     const int64_t H = pop.holes, S = pop.surplus;
     PopPlan pl = {};
-    pl.holes = H;
-    pl.surplus = S;
     pl.alive = cp.nMain - H + S;
     pl.remove = S > H ? S - H : 0;
     const double R = (double)pl.remove;
@@ -1098,7 +1096,6 @@ __device__ bool radix_threshold(PopLds& L, const CondParams& cp, int64_t K, int6
 // needs five passes.  Every thread gets the plan's threshold, or the status.
 __device__ void removal_threshold(const CondParams& cp, int64_t K, PopPlan& pl, PopLds& L) {
     const int64_t R = pl.remove;
-    pl.marks = K;
     if (K < R || K > 0xffffffffLL) {
         pl.status |= ST_POPCTL;
         return;
@@ -1570,7 +1567,7 @@ __global__ __launch_bounds__(kBlock) void k_hist(DevState<V> s, const SlotRange*
 }
 
 // ----------------------------------------------------------------- finish
-// summary[c] = [ event record (3P + 8) | moment sums (kMomentRecord) | plan (8) ]
+// summary[c] = [ event record (3P + 8) | moment sums (kMomentRecord) | status ]
 // Chunk records are summed in a fixed order: thread (r, f) of a block adds
 // field f of records r, r + kFinishRows, ... in order (neighbouring threads
 // read neighbouring fields), then thread f adds the rows.  The integer
@@ -1655,13 +1652,7 @@ __global__ __launch_bounds__(kFinishBlock) void k_finish(DevWork w, int P) {
         w.accLoss[i] = 0;
     }
     if (threadIdx.x == 0) {
-        const CondPop pop = pop_total(w, c);
-        const PopPlan pl = plan_of(pop, cp);
-        double* tail = out + R + kMomentRecord;
-        tail[0] = (double)pl.holes; tail[1] = (double)pl.surplus; tail[2] = (double)pl.alive;
-        tail[3] = (double)pl.remove; tail[4] = (double)pop.marks; tail[5] = 0;
-        tail[6] = (double)w.status[c];
-        tail[7] = 0;
+        out[R + kMomentRecord] = (double)w.status[c];
         for (int k = 0; k < kPopCopies; ++k) w.pop[(size_t)k * w.popStride + c] = CondPop{};
     }
 }

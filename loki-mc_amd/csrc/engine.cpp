@@ -8,8 +8,8 @@
 // histogram sums and their re-binning (BoltzmannMC.C:1492-1548), and the time
 // averages (BoltzmannMC.C:1484-1741, 1950-2266).  Electrons, flights,
 // collisions, population control and all per-electron reductions live on the
-// GPU (kernels.hip); one interval of every running condition is one batch of
-// launches followed by one small device-to-host copy of per-condition sums.
+// GPU (kernels.hip); one interval of a part of the running conditions is one batch
+// of launches, whose last kernel writes the per-condition sums to pinned host memory.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

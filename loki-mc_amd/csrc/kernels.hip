@@ -49,15 +49,16 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 // kernel: a null event costs a flight and a null test, not a whole step of
 // the wave's bookkeeping.  Measured per interval on the 64-condition scan,
 // mixed form: 1 / 2 / 3 / 4 events, 0.981 / 0.963 / 0.989 / 1.062 ms (longer
-// runs leave more lanes idle in the loop than they save); FP64 form: 1 / 2
-// events, 1.596 / 1.663 ms.
+// runs leave more lanes idle in the loop than they save); FP64 form, whose flights
+// are the longer: 1 / 2 events, 1.419 / 1.434 ms, one condition of 3e7 electrons
+// 2106 / 2122 us, four ECR conditions 76.3 / 77.7, one of 1e5 67.5 / 66.3.
 template <typename V> constexpr int null_run() { return sizeof(V) == 8 ? 1 : 2; }
 
 // LDS of one wave of the flight kernel: collision tallies [3P] (64-bit), the
 // histogram grid of the chunk's condition [8] (FP64), the null-test envelope
 // [2 kEnvBins] (V) and the EEDF counts of a histogram taken at load [histLds]
-// (16-bit, two cells per word: a chunk holds at most 65535 main electrons)
-// (32-bit).  The record ring is a separate static array.
+// (16-bit, two cells per word: a chunk holds at most 65535 main electrons).
+// The record ring is a separate static array.
 template <typename V> __host__ __device__ constexpr size_t flight_wave_lds(int P, int histLds) {
     return (size_t)3 * P * 8 + 8 * 8 + (size_t)2 * kEnvBins * sizeof(V) + (size_t)((histLds + 1) / 2) * 4;
 }
@@ -593,8 +594,11 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
     wave_lds_sync();
 
     // two record pieces per ring load, except with the cylindrical histograms
-    // counted at load: there the pairs raised the flight kernel from 163 to
-    // 169 VGPRs, past the 168 of three waves per SIMD
+    // counted at load: six VGPRs more there (mixed 130 -> 136 in DC, but AC+B 164 -> 170,
+    // past the 168 of three waves per SIMD), for no gain where they fit: flight
+    // kernel per interval, pairs against single pieces, one condition of 1e5 electrons
+    // in FP64 67.7 / 67.5 us, eight of 1e5 150.5 / 150.0, 24 AC conditions of 2e5
+    // 664 / 664
     constexpr bool kPairFill = HIST != HIST_LDS_CYL;
     const int count = ch.count;
     int nextMain = 0, nq = 0, nextNew = 0, holes = 0;
@@ -820,9 +824,10 @@ __device__ __forceinline__ void advance_chunk(const DevState<V>& s, const DevWor
     wave_lds_sync();
 }
 
-// Waves per SIMD the flight kernel is compiled for.  FP64: two (172-187 VGPRs;
+// Waves per SIMD the flight kernel is compiled for.  FP64: two (172-210 VGPRs;
 // its record rings leave the LDS room for two blocks per CU anyway).  Mixed form:
-// the compiler's choice (136-168 VGPRs, three waves).  More waves do not make
+// the compiler's choice (130-168 VGPRs, three waves; two for AC+B off resonance with
+// thermal targets and no cylindrical condition, at 173).  More waves do not make
 // either faster: with a ring of 80 records and an FP32 envelope, so that the LDS
 // held them, one condition of 3e7 electrons took 2416 us per interval with three
 // FP64 waves against 2354 with two, and 1515 with four mixed waves against 1389
@@ -956,8 +961,9 @@ __device__ __forceinline__ bool mark_alive(const uint8_t* alive, const Chunk& ch
 // loads of its results.  Per interval, in the blocks against with k_plan_marks:
 // one condition of 1e4 electrons 8.3 us against 6.1 + 6.9, one of 1e5 11.6
 // against 6.4 + 6.5, eight of 1e5 at up to 500 Td (2 % newborns) 31 against
-// 10.3 + 10.3, the 64-condition scan with half of its conditions planned in the
-// blocks 67 + 18 against 30 + 17.
+// 10.3 + 10.3.  It does not pay beside larger conditions, for which k_plan_marks is
+// launched all the same: the 64-condition scan with half of its conditions planned in
+// the blocks 67 + 18 against 30 + 17.
 __host__ __device__ __forceinline__ bool plans_direct(const CondParams& cp) { return cp.nMain <= kPlanDirect; }
 
 // The marks of each chunk of a condition with removals, counted per lane and

@@ -249,6 +249,15 @@ double max_accel_energy(const Cond& c, double initialEnergy, double deltaT) {
 constexpr int kMaxParts = 2;
 constexpr int64_t kPartElectrons = 400000;
 constexpr int kPartShare = 7;
+// The parts' streams have to be on different hardware queues: where streams made and
+// freed before the engine leave one queue with far fewer of them than the others, two
+// new streams in a row are put there, and two parts in turn are slower than one
+// (64-condition scan, mixed, two parts beside each other, in turn, and one part: 15.8,
+// 21.1, 19.9 ms; eight conditions of 1e5 6.7, 10.1, 9.1; 24 AC conditions 11.0, 14.9, 13.9;
+// one part as of the build before there were two).  So a second stream is taken
+// that is seen to run beside the first; those that are not stay until then, so that the
+// next one goes elsewhere.  Without one in kStreamTries the batch runs in one part.
+constexpr int kStreamTries = 8;
 
 // =============================================================== Engine<V>
 template <typename V> class Engine : public EngineBase {
@@ -769,26 +778,53 @@ public:
         return EKMC_OK;
     }
 
+    // A stream whose kernels run beside those of `stream`, or null.
+    ekmc_status stream_beside(hipStream_t* out) {
+        hipStream_t tried[kStreamTries] = {};
+        hipError_t e = hipSuccess;
+        *out = nullptr;
+        int n = 0;
+        while (n < kStreamTries && !*out && e == hipSuccess) {
+            bool beside = false;
+            e = hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking);
+            if (e != hipSuccess) break;
+            e = run_beside(stream, tried[n], queue.p, &beside);
+            if (beside) *out = tried[n];
+            ++n;
+        }
+        for (int k = 0; k < n; ++k)
+            if (tried[k] != *out) (void)hipStreamDestroy(tried[k]);
+        if (e == hipSuccess) e = hipMemsetAsync(queue.p, 0, 2 * sizeof(uint32_t), stream);
+        if (e != hipSuccess && *out) {
+            (void)hipStreamDestroy(*out);
+            *out = nullptr;
+        }
+        HIP_TRY(e);
+        return EKMC_OK;
+    }
+
     // The parts of the batch: two of about as many electrons where the batch
-    // has kPartElectrons, else one.
+    // has kPartElectrons and a second stream runs beside the first, else one.
     ekmc_status create_parts(const std::vector<SlotRange>& hr) {
         std::vector<int> cut = {0, nCond};
+        hipStream_t second = nullptr;
         if (nCond > 1 && totalMain >= kPartElectrons && timerLevel < 2) {
+            ekmc_status st = stream_beside(&second);
+            if (st != EKMC_OK) return st;
+        }
+        if (second) {
             int64_t sum = 0;
             int c = 0;
             while (c + 1 < nCond && 2 * (sum + hcp[c].nMain / 2) < totalMain) sum += hcp[c++].nMain;
             cut.insert(cut.begin() + 1, std::max(c, 1));
         }
         parts.resize(cut.size() - 1);
+        parts[0].stream = stream;
+        if (second) parts[1].stream = second;  // the engine's from here on
         for (size_t i = 0; i < parts.size(); ++i) {
             Part& p = parts[i];
             p.c0 = cut[i];
             p.c1 = cut[i + 1];
-            p.stream = stream;
-            if (i > 0) {
-                p.stream = nullptr;
-                HIP_TRY(hipStreamCreateWithFlags(&p.stream, hipStreamNonBlocking));
-            }
             // times only: nothing waits on them for memory
             for (int k = 0; k < K_COUNT; ++k) {
                 HIP_TRY(hipEventCreateWithFlags(&p.timer.start[k], hipEventReleaseToDevice));

@@ -269,6 +269,11 @@ template <typename V> constexpr size_t flight_ring_lds() {
     return (size_t)ring_segs<V>() * (kBlock / kWave) * kRingSeg * sizeof(Rec<V>);
 }
 
+// Whether kernels launched on the streams a and b run at the same time: HIP's streams
+// share a few hardware queues, and those that share one run in turn.  `word` is two
+// words of device memory.  Both streams are idle afterwards.
+hipError_t run_beside(hipStream_t a, hipStream_t b, uint32_t* word, bool* beside);
+
 template <typename V>
 hipError_t launch_op_accelerate(const CondParams* cond, int64_t n, const double* time, const double* dt,
                                 double* pos, double* vel, double* energy, double* gain, hipStream_t st);

@@ -1855,6 +1855,20 @@ __global__ __launch_bounds__(kBlock) void k_op_philox(int64_t n, const uint32_t*
     for (int k = 0; k < 4; ++k) out[4 * i + k] = c[k];
 }
 
+// Whether kernels of two streams run at the same time: one waits for the other's
+// word, for at most a millisecond or so (word[0] the signal, word[1] the answer).
+constexpr int kBesidePolls = 1000;
+__global__ void k_await(uint32_t* word) {
+    for (int k = 0; k < kBesidePolls; ++k) {
+        if (atomicAdd(&word[0], 0u) != 0) {
+            word[1] = 1;
+            return;
+        }
+        __builtin_amdgcn_s_sleep(16);
+    }
+}
+__global__ void k_signal(uint32_t* word) { atomicExch(&word[0], 1u); }
+
 // ------------------------------------------------------------- launchers
 static inline unsigned chunk_grid(int nChunks) { return (unsigned)((nChunks + kWavesPerBlock - 1) / kWavesPerBlock); }
 // Dynamic LDS of a flight-kernel block: the process records [P], then the
@@ -2012,6 +2026,29 @@ hipError_t launch_op_collide(const CondParams* cond, const DevProcesses& pr, con
     hipLaunchKernelGGL(k_op_collide<V>, dim3(grid_of(n)), dim3(kBlock), 0, st, cond, pr, tables, n, vel, energy,
                        nue, variates, pid, ejv, eje, de);
     return hipGetLastError();
+}
+
+hipError_t run_beside(hipStream_t a, hipStream_t b, uint32_t* word, bool* beside) {
+    uint32_t answer = 0;
+    hipError_t e = hipSuccess;
+    // the first turn only brings the streams into being on the device
+    for (int turn = 0; turn < 2 && e == hipSuccess; ++turn) {
+        e = hipMemsetAsync(word, 0, 2 * sizeof(uint32_t), a);
+        if (e == hipSuccess) e = hipStreamSynchronize(a);
+        if (e == hipSuccess && turn == 1) {
+            hipLaunchKernelGGL(k_await, dim3(1), dim3(1), 0, a, word);
+            e = hipGetLastError();
+        }
+        if (e == hipSuccess) {
+            hipLaunchKernelGGL(k_signal, dim3(1), dim3(1), 0, b, word);
+            e = hipGetLastError();
+        }
+        const hipError_t ea = hipStreamSynchronize(a), eb = hipStreamSynchronize(b);
+        if (e == hipSuccess) e = ea != hipSuccess ? ea : eb;
+    }
+    if (e == hipSuccess) e = hipMemcpy(&answer, word + 1, sizeof(answer), hipMemcpyDeviceToHost);
+    *beside = e == hipSuccess && answer != 0;
+    return e;
 }
 
 hipError_t launch_op_philox(int64_t n, const uint32_t* ctr, const uint32_t* key, uint32_t* out, hipStream_t st) {
